@@ -370,6 +370,13 @@ int sfl_rmsnorm_rows_scaled(const float* x, const void* w, void* act_xg, float* 
 int sfl_gemm_residual_norm(const void* a, const void* w, float* x, int m, int n, int k, const void* gain_next,
                            void* act_xg, float* ss_parts, int dtype, void* stream);
 
+/* The same with parts of `part` features (ceil(n / part) of them): 128, or
+ * sfl_gemm_norm_part(m, n, k), the part size of the tile this shape runs on (32
+ * for the small tiles of short prompts, which 128 would exclude). */
+int sfl_gemm_norm_part(int m, int n, int k);
+int sfl_gemm_residual_norm_parts(const void* a, const void* w, float* x, int m, int n, int k, const void* gain_next,
+                                 void* act_xg, float* ss_parts, int part, int dtype, void* stream);
+
 /* rscale[r] = 1 / sqrt(sum_p ss_parts[p][r] / d_model + 1e-5), parts summed in order. */
 int sfl_norm_scale(const float* ss_parts, int parts, int m, int d_model, float* rscale, void* stream);
 
@@ -383,6 +390,14 @@ int sfl_gemm_qkv_rope_scaled(const void* a_xg, const void* w_qkv, const float* r
  * before silu(.) * (.). */
 int sfl_gemm_swiglu_scaled(const void* a_xg, const void* w13_interleaved, const float* rscale, void* h_out,
                            int m, int d_ff, int k, int dtype, void* stream);
+
+/* The same two with the scales formed in the kernel from the parts a residual
+ * GEMM left (the sums and bits of sfl_norm_scale, without its launch). */
+int sfl_gemm_qkv_rope_normed(const void* a_xg, const void* w_qkv, const float* ss_parts, int parts, int m, int seq,
+                             int d_model, int heads, const float* cos_t, const float* sin_t, void* q_out,
+                             void* k_cache, void* v_cache, int capacity, int dtype, void* stream);
+int sfl_gemm_swiglu_normed(const void* a_xg, const void* w13_interleaved, const float* ss_parts, int parts,
+                           void* h_out, int m, int d_ff, int k, int dtype, void* stream);
 
 #ifdef __cplusplus
 }

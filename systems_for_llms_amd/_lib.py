@@ -49,9 +49,13 @@ SIGNATURES: dict[str, list] = {
     "sfl_rmsnorm_rows": [P, P, P, c_int, c_int, c_int, c_int, P],
     "sfl_rmsnorm_rows_scaled": [P, P, P, P, c_int, c_int, c_int, P],
     "sfl_gemm_residual_norm": [P, P, P, c_int, c_int, c_int, P, P, P, c_int, P],
+    "sfl_gemm_norm_part": [c_int, c_int, c_int],
+    "sfl_gemm_residual_norm_parts": [P, P, P, c_int, c_int, c_int, P, P, P, c_int, c_int, P],
     "sfl_norm_scale": [P, c_int, c_int, c_int, P, P],
     "sfl_gemm_qkv_rope_scaled": [P, P, P, c_int, c_int, c_int, c_int, P, P, P, P, P, c_int, c_int, P],
     "sfl_gemm_swiglu_scaled": [P, P, P, P, c_int, c_int, c_int, c_int, P],
+    "sfl_gemm_qkv_rope_normed": [P, P, P, c_int, c_int, c_int, c_int, c_int, P, P, P, P, P, c_int, c_int, P],
+    "sfl_gemm_swiglu_normed": [P, P, P, c_int, P, c_int, c_int, c_int, c_int, P],
     "sfl_causal_attention_f32": [P, P, P, P, c_int, c_int, c_int, c_int, POINTER(c_long), POINTER(c_long),
                                  POINTER(c_long), POINTER(c_long), c_float, P],
 }

@@ -20,211 +20,18 @@
 //             position m % T, q to [B, H, T, dk] bf16, k/v to the KV cache.
 //   SWIGLU    W is W1/W3 interleaved in blocks of 8 rows; h = silu(a) * c
 //             (layers.py:114-115) as bf16 [M, d_ff].
-#include "attn_mfma.hpp"
+#include <algorithm>
+#include <initializer_list>
+
+#include "gemm16.hpp"
 #include "gemm_f32.hpp"
-#include "lds_dma.hpp"
 
 namespace sfl {
 namespace {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
 constexpr int TN = 128, TM = 128, TK = 64;
 constexpr int LDT = TK + 8;      // LDS row stride (elements)
 constexpr int kThreads = 256;
-
-enum GemmEpi { G_PLAIN = 0, G_QKV = 1, G_SWIGLU = 2 };
-
-struct GemmArgs {
-  const uint16_t* a;   // [M, K]
-  const uint16_t* w;   // [N, K]
-  int m, n, k;
-  // PLAIN
-  void* c;             // [M, N] (ldc = N)
-  int c_f32, accumulate;
-  // QKV
-  const float* cos_t;
-  const float* sin_t;
-  int seq, heads, head_dim, d_model, cap;
-  uint16_t* q_out;     // [B, H, T, dk]
-  uint16_t* k_cache;   // [B, H, cap, dk]
-  uint16_t* v_cache;
-  // SWIGLU
-  uint16_t* h_out;     // [M, N/2]
-  // PLAIN residual (fp32 C += A W^T) that also prepares the next RMSNorm
-  // (norm_gain null: not): norm_act = bf16(C * gain), and per token and
-  // 128-feature part the sum of C^2 in norm_ss [ceil(N / 128)][M].
-  const uint16_t* norm_gain;
-  uint16_t* norm_act;
-  float* norm_ss;
-  // QKV / SWIGLU fed by such an input: the products are scaled by
-  // row_scale[m] = 1 / rms of token m (null: not).
-  const float* row_scale;
-  // Every bf16 output base is 16-byte aligned: the 32x32 kernel then stores
-  // 8 consecutive outputs per lane (lane pairs exchange halves first).
-  int vec16;
-};
-
-template <typename T>
-__device__ __forceinline__ f32x4 mfma16(const u32x4& a, const u32x4& b, f32x4 c);
-template <>
-__device__ __forceinline__ f32x4 mfma16<bf16_t>(const u32x4& a, const u32x4& b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-template <>
-__device__ __forceinline__ f32x4 mfma16<f16_t>(const u32x4& a, const u32x4& b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-}
-
-// One value rounded to T (round to nearest even), as raw bits.
-template <typename T> __device__ __forceinline__ uint16_t bits16(float v);
-template <> __device__ __forceinline__ uint16_t bits16<bf16_t>(float v) { return f32_to_bf16_bits(v); }
-template <> __device__ __forceinline__ uint16_t bits16<f16_t>(float v) { return f32_to_f16_bits(v); }
-
-// The low and high T values of a packed pair, as fp32.
-template <typename T> __device__ __forceinline__ float lo16(uint32_t w);
-template <typename T> __device__ __forceinline__ float hi16(uint32_t w);
-template <> __device__ __forceinline__ float lo16<bf16_t>(uint32_t w) { return bf16_lo(w); }
-template <> __device__ __forceinline__ float hi16<bf16_t>(uint32_t w) { return bf16_hi(w); }
-template <> __device__ __forceinline__ float lo16<f16_t>(uint32_t w) { return f16_bits_to_f32(uint16_t(w & 0xffffu)); }
-template <> __device__ __forceinline__ float hi16<f16_t>(uint32_t w) { return f16_bits_to_f32(uint16_t(w >> 16)); }
-
-// v, or zeros when !keep. Selected per component: a select of whole uint4
-// structs is lowered through scratch memory.
-__device__ __forceinline__ uint4 keep16(const uint4& v, bool keep) {
-  return make_uint4(keep ? v.x : 0u, keep ? v.y : 0u, keep ? v.z : 0u, keep ? v.w : 0u);
-}
-
-
-// Where a lane's 4 QKV features and its token go: section (0 q, 1 k, 2 v),
-// head, dim of the first feature; batch row and position of the token.
-// Computed once per feature tile / token tile by the caller (integer
-// divisions by runtime sizes are long instruction sequences).
-struct QkvFeat { int section, head, dim; };
-struct QkvTok { int b, t; };
-
-__device__ __forceinline__ QkvFeat qkv_feat(const GemmArgs& g, int n) {
-  const int section = n / g.d_model;
-  const int f = n - section * g.d_model;
-  const int head = f / g.head_dim;
-  return QkvFeat{section, head, f - head * g.head_dim};
-}
-// qkv_feat of feature nt + off from base = qkv_feat(nt), 0 <= off < 32: the
-// head changes at most twice within 32 features (head dims >= 16), so two
-// compare-and-wrap steps replace the two integer divisions.
-__device__ __forceinline__ QkvFeat qkv_feat_at(const GemmArgs& g, const QkvFeat& base, int off) {
-  QkvFeat f{base.section, base.head, base.dim + off};
-#pragma unroll
-  for (int w = 0; w < 2; ++w) {
-    if (f.dim >= g.head_dim) {
-      f.dim -= g.head_dim;
-      if (++f.head == g.heads) {
-        f.head = 0;
-        ++f.section;
-      }
-    }
-  }
-  return f;
-}
-__device__ __forceinline__ QkvTok qkv_tok(const GemmArgs& g, int m) {
-  const int b = m / g.seq;
-  return QkvTok{b, m - b * g.seq};
-}
-
-// RoPE (attention.py:44-58) of 4 consecutive q or k features (dims dim ..
-// dim+3 of one head: two rotation pairs) of token qt; v features pass through.
-__device__ __forceinline__ void rope4(const GemmArgs& g, float (&y)[4], const QkvFeat& qf, const QkvTok& qt) {
-  if (qf.section >= 2) return;
-  // Feature-major tables [head_dim / 2][cap]: the 32 lanes of a group hold 32
-  // consecutive tokens, so each load reads consecutive floats (row-major
-  // tables put the 32 tokens on 32 cache lines: 345 -> 330 us on the 324M
-  // q/k/v shape, same values).
-  const long r0 = long(qf.dim / 2) * g.cap + qt.t;
-  const float2 c = make_float2(g.cos_t[r0], g.cos_t[r0 + g.cap]);
-  const float2 s = make_float2(g.sin_t[r0], g.sin_t[r0 + g.cap]);
-  const float e0 = y[0], o0 = y[1], e1 = y[2], o1 = y[3];
-  y[0] = e0 * c.x - o0 * s.x;
-  y[1] = e0 * s.x + o0 * c.x;
-  y[2] = e1 * c.y - o1 * s.y;
-  y[3] = e1 * s.y + o1 * c.y;
-}
-
-// Destination of feature qf of token qt: q [B, H, T, dk] or the k / v cache [B, H, cap, dk].
-__device__ __forceinline__ uint16_t* qkv_dst(const GemmArgs& g, const QkvFeat& qf, const QkvTok& qt) {
-  if (qf.section == 0) return g.q_out + ((long(qt.b) * g.heads + qf.head) * g.seq + qt.t) * g.head_dim + qf.dim;
-  uint16_t* cache = qf.section == 1 ? g.k_cache : g.v_cache;
-  return cache + ((long(qt.b) * g.heads + qf.head) * g.cap + qt.t) * g.head_dim + qf.dim;
-}
-
-// silu(a) * c = a * c / (1 + e^-a) with the hardware base-2 exponential and
-// reciprocal (e^-a = 2^(-a log2 e); each ~1 ulp): the bf16 rounding of the
-// result dominates their error. a -> -inf gives 2^+inf = inf and a zero
-// reciprocal (a signed zero), as the exact form does.
-__device__ __forceinline__ float silu_mul(float a, float c) {
-  const float e = __builtin_amdgcn_exp2f(a * -1.4426950408889634f);
-  return a * c * __builtin_amdgcn_rcpf(1.f + e);
-}
-
-// Two packed groups of 4 bf16 outputs, A (lane-local features f .. f+3) and
-// B (f+8 .. f+11), where lane l ^ 32 holds f+4 .. f+7 and f+12 .. f+15: one
-// v_permlane32_swap per dword gives lanes 0..31 features f .. f+7 (own A,
-// partner's A) and lanes 32..63 features f+8 .. f+15 (partner's B, own B),
-// one 16-byte store each instead of two 8-byte stores.
-__device__ __forceinline__ uint4 pair8(const uint32_t (&a)[2], const uint32_t (&b)[2]) {
-  const auto s0 = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false);
-  const auto s1 = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
-  return make_uint4(s0[0], s1[0], s0[1], s1[1]);
-}
-
-// Epilogue of one 16x16 MFMA tile: v holds features nt + 4*grp + (0..3) of
-// token m. Every lane must call it (the SwiGLU pairing shuffles).
-template <typename T, int E>
-__device__ __forceinline__ void store_tile(const GemmArgs& g, const f32x4& v, int nt, int grp, int m,
-                                           QkvFeat qf = QkvFeat{}, QkvTok qt = QkvTok{}) {
-  const int n = nt + 4 * grp;
-  float y[4] = {v[0], v[1], v[2], v[3]};
-  if constexpr (E == G_SWIGLU) {
-    // Rows 0..7 of the 16-row tile are W1 features, rows 8..15 the
-    // matching W3 features: lane groups 0,1 pair with groups 2,3.
-    float c3[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) c3[e] = lane_xor(y[e], 32);
-    if (grp >= 2 || m >= g.m) return;
-    const int f = nt / 2 + 4 * grp;  // hidden feature index
-    if (f >= g.n / 2) return;
-    float h[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) h[e] = silu_mul(y[e], c3[e]);
-    *reinterpret_cast<uint2*>(g.h_out + long(m) * (g.n / 2) + f) = make_uint2(pack2<T>(h[0], h[1]), pack2<T>(h[2], h[3]));
-  } else {
-    if (m >= g.m || n >= g.n) return;
-    if constexpr (E == G_PLAIN) {
-      if (g.c_f32) {
-        float* c = static_cast<float*>(g.c) + long(m) * g.n + n;
-        if (n + 3 < g.n && (g.n & 3) == 0) {
-          float4 old = g.accumulate ? *reinterpret_cast<const float4*>(c) : make_float4(0.f, 0.f, 0.f, 0.f);
-          *reinterpret_cast<float4*>(c) = make_float4(old.x + y[0], old.y + y[1], old.z + y[2], old.w + y[3]);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (n + e < g.n) c[e] = (g.accumulate ? c[e] : 0.f) + y[e];
-        }
-      } else {
-        uint16_t* c = static_cast<uint16_t*>(g.c) + long(m) * g.n + n;
-        if (n + 3 < g.n && (g.n & 3) == 0) {
-          *reinterpret_cast<uint2*>(c) = make_uint2(pack2<T>(y[0], y[1]), pack2<T>(y[2], y[3]));
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (n + e < g.n) c[e] = bits16<T>(y[e]);
-        }
-      }
-    } else {  // G_QKV
-      rope4(g, y, qf, qt);
-      *reinterpret_cast<uint2*>(qkv_dst(g, qf, qt)) = make_uint2(pack2<T>(y[0], y[1]), pack2<T>(y[2], y[3]));
-    }
-  }
-}
 
 template <typename T, int E>
 __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmArgs g) {
@@ -320,49 +127,6 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmArgs g) {
 // free of bank conflicts. Rows past the matrix read as zeros through the
 // buffer range check. K advances by 64 through two LDS stages, the loads of
 // the next step in flight while a step computes.
-constexpr int K2 = 64;     // K step
-constexpr int TB = 128;    // features and tokens per workgroup
-
-
-template <int TN_, int TM_, int SL_>
-struct Stage32 {
-  uint4 w[TN_][SL_];  // [row][swizzled 16-byte slot]
-  uint4 a[TM_][SL_];
-};
-
-// Physical 16-byte slot offset of row r in a stage of SL slots per row: the
-// XOR under which the MFMA operand reads (16 consecutive lanes reading rows r
-// .. r+15 at one logical slot, 256 bytes per LDS cycle) touch every bank
-// once. Rows of 128 bytes already alternate bank halves, rows of 64 bytes
-// cycle through bank quarters, so the swizzle only has to separate rows that
-// share a half / quarter.
-template <int SL>
-__device__ __forceinline__ int stage_swizzle(int r) {
-  return SL == 8 ? (r >> 1) & 7 : (r >> 2) & 3;
-}
-
-// Tile of workgroup b in a 1-D grid of tn x tm tiles, XCD-aware: workgroups
-// are dealt to the 8 XCDs round-robin (b % 8) and each XCD has its own L2, so
-// XCD x is given a contiguous range of the tile order, and that order walks
-// groups of kGroupM token tiles across the feature tiles. The workgroups an
-// XCD runs at once then cover about 4 token tiles x 8 feature tiles, whose
-// operands stay in (or near) its 4 MB L2 (for 256 x 384 tiles, 448 KB of the
-// 2.5 MB a K step requests are distinct).
-constexpr int kXcds = 8;
-constexpr int kGroupM = 4;
-
-__device__ __forceinline__ int2 xcd_tile(int b, int tn, int tm) {
-  const int total = tn * tm;
-  const int x = b % kXcds, idx = b / kXcds;
-  const int base = total / kXcds, extra = total % kXcds;  // XCD x gets base + (x < extra) tiles
-  const int t = x * base + min(x, extra) + idx;
-  const int group = t / (kGroupM * tn);
-  const int gm0 = group * kGroupM;
-  const int gsize = min(kGroupM, tm - gm0);
-  const int r = t - group * kGroupM * tn;
-  return make_int2(r / gsize, gm0 + r % gsize);  // (feature tile, token tile)
-}
-
 // TBN x TBM tiles (features x tokens) per workgroup of WN x WM waves; a wave
 // owns (TBN/WN) x (TBM/WM) as blocks of 32 x 32. 128 x 128 with 2 x 2 waves:
 // two workgroups per CU (64 KB of LDS each), 64 x 64 per wave. 256 x 384 with
@@ -491,11 +255,14 @@ void gemm32_kernel(GemmArgs g) {
 #pragma unroll
   for (int p = 0; p < NS - 1; ++p)
     if (p < ksteps) SFL_G32_ISSUE(st[p], p)
+  if constexpr (E != G_PLAIN) {
+    if (g.ss) {
+#pragma unroll
+      for (int j = 0; j < NBM; ++j) rsc[j] = parts_scale(g, min(m0 + (TBM / WM) * wm + 32 * j + l32, g.m - 1));
+    }
+  }
   for (int kt = 0; kt < ksteps; ++kt) {
-    const int younger = min(NS - 2, ksteps - 1 - kt);  // stages issued after stage kt
-    if (NS > 3 && younger >= 2) __builtin_amdgcn_s_waitcnt(sfl_vmcnt(NS > 3 ? 2 * CPW : 0));
-    else if (NS > 2 && younger >= 1) __builtin_amdgcn_s_waitcnt(sfl_vmcnt(NS > 2 ? CPW : 0));
-    else __builtin_amdgcn_s_waitcnt(sfl_vmcnt(0));
+    wait_younger<NS - 2, CPW>(min(NS - 2, ksteps - 1 - kt));  // stages issued after stage kt
     __syncthreads();  // every wave's loads of this stage landed; stage (kt - 1) % NS is no longer read
     if (kt + NS - 1 < ksteps) SFL_G32_ISSUE(st[(kt + NS - 1) % NS], kt + NS - 1)
     SFL_G32_COMPUTE(st[kt % NS])
@@ -505,7 +272,6 @@ void gemm32_kernel(GemmArgs g) {
 
   if constexpr (E == G_PLAIN) {
     if (acc_c) {
-      float* const c = static_cast<float*>(g.c);
       const bool norm = g.norm_gain != nullptr;  // uniform
       // The next norm's gains for this lane's features (one batch of loads,
       // before any store).
@@ -524,40 +290,8 @@ void gemm32_kernel(GemmArgs g) {
         const int m = m0 + (TBM / WM) * wm + 32 * j + l32;
         ssq[j] = 0.f;
 #pragma unroll
-        for (int i = 0; i < NBN; ++i) {
-          const int nt = n0 + (TBN / WN) * wn + 32 * i;
-          uint32_t pk[4][2];  // T(x * gain) of features nt + 8q + 4hf + (0..3)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int n = nt + 8 * q + 4 * hf;
-            const float4 v = make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
-                                         acc[i][j][4 * q + 3]);
-            const bool in = m < g.m && n < g.n;
-            if (in) *reinterpret_cast<float4*>(c + long(m) * g.n + n) = v;
-            if (norm) {
-              pk[q][0] = pack2<T>(v.x * lo16<T>(gw[i][q].x), v.y * hi16<T>(gw[i][q].x));
-              pk[q][1] = pack2<T>(v.z * lo16<T>(gw[i][q].y), v.w * hi16<T>(gw[i][q].y));
-              if (in) ssq[j] += (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
-            }
-          }
-          if (norm) {
-            if (g.vec16) {  // 8 consecutive features per lane (every lane swaps)
-#pragma unroll
-              for (int q = 0; q < 4; q += 2) {
-                const uint4 o = pair8(pk[q], pk[q + 1]);
-                const int n = nt + 8 * q + 8 * hf;
-                if (m < g.m && n < g.n) *reinterpret_cast<uint4*>(g.norm_act + long(m) * g.n + n) = o;
-              }
-            } else {
-#pragma unroll
-              for (int q = 0; q < 4; ++q) {
-                const int n = nt + 8 * q + 4 * hf;
-                if (m < g.m && n < g.n)
-                  *reinterpret_cast<uint2*>(g.norm_act + long(m) * g.n + n) = make_uint2(pk[q][0], pk[q][1]);
-              }
-            }
-          }
-        }
+        for (int i = 0; i < NBN; ++i)
+          residual_block<T>(g, acc[i][j], n0 + (TBN / WN) * wn + 32 * i, m, hf, norm, gw[i], ssq[j]);
       }
       if (norm) {
         // Sum of squares per token over each 128-feature part: this lane's 32
@@ -592,102 +326,8 @@ void gemm32_kernel(GemmArgs g) {
     const int m = m0 + (TBM / WM) * wm + 32 * j + l32;
     const QkvTok tok = E == G_QKV ? qkv_tok(g, m) : QkvTok{};
 #pragma unroll
-    for (int i = 0; i < NBN; ++i) {
-      const int nt = n0 + (TBN / WN) * wn + 32 * i;
-      // One division pair per 32-feature block; the lane's features derive from
-      // it. With head dims that are multiples of 32 the block is one head of one
-      // section: its features share the destination row.
-      const QkvFeat fb = E == G_QKV ? qkv_feat(g, nt) : QkvFeat{};
-      const bool blk = E == G_QKV && g.head_dim % 32 == 0;
-      uint16_t* const base = blk ? qkv_dst(g, fb, tok) : nullptr;
-      if constexpr (E == G_SWIGLU) {
-        // W1/W3 interleaved in blocks of 8 rows: groups q = 0, 2 are W1 features,
-        // q + 1 the matching W3 features, all in this lane. Hidden features
-        // nt/2 + 4q + 4hf .. +3; with vec16 the two groups go out as one
-        // 16-byte store per lane at nt/2 + 8hf (d_ff % 8 == 0: a group of 8 is
-        // wholly inside or outside d_ff).
-        uint32_t pk[2][2];
-#pragma unroll
-        for (int q = 0; q < 4; q += 2) {
-          float h[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float a1 = acc[i][j][4 * q + e] * rsc[j], a3 = acc[i][j][4 * q + 4 + e] * rsc[j];
-            h[e] = silu_mul(a1, a3);
-          }
-          pk[q / 2][0] = pack2<T>(h[0], h[1]);
-          pk[q / 2][1] = pack2<T>(h[2], h[3]);
-        }
-        if (g.vec16) {
-          const uint4 v8 = pair8(pk[0], pk[1]);
-          const int f = nt / 2 + 8 * hf;
-          if (m < g.m && f < g.n / 2) *reinterpret_cast<uint4*>(g.h_out + long(m) * (g.n / 2) + f) = v8;
-        } else if (m < g.m) {
-#pragma unroll
-          for (int q = 0; q < 4; q += 2) {
-            const int f = nt / 2 + 4 * q + 4 * hf;  // hidden feature index
-            if (f < g.n / 2)
-              *reinterpret_cast<uint2*>(g.h_out + long(m) * (g.n / 2) + f) = make_uint2(pk[q / 2][0], pk[q / 2][1]);
-          }
-        }
-      } else if (E != G_PLAIN || (!g.c_f32 && !g.accumulate)) {
-        // bf16 outputs (q/k/v, plain bf16): feature groups q and q + 1 of the
-        // lane pair go out as 16-byte stores (vec16; whole 32-feature blocks
-        // inside N), else 8 bytes per group.
-        const bool wide = g.vec16 && nt + 32 <= g.n && (E == G_QKV || g.n % 8 == 0);
-#pragma unroll
-        for (int q = 0; q < 4; q += 2) {
-          uint32_t pk[2][2];
-          QkvFeat feat[2];
-#pragma unroll
-          for (int r = 0; r < 2; ++r) {
-            float y[4] = {acc[i][j][4 * (q + r)] * rsc[j], acc[i][j][4 * (q + r) + 1] * rsc[j],
-                          acc[i][j][4 * (q + r) + 2] * rsc[j], acc[i][j][4 * (q + r) + 3] * rsc[j]};
-            feat[r] = E != G_QKV ? QkvFeat{}
-                      : blk ? QkvFeat{fb.section, fb.head, fb.dim + 8 * (q + r) + 4 * hf}
-                            : qkv_feat_at(g, fb, 8 * (q + r) + 4 * hf);
-            if constexpr (E == G_QKV) rope4(g, y, feat[r], tok);
-            pk[r][0] = pack2<T>(y[0], y[1]);
-            pk[r][1] = pack2<T>(y[2], y[3]);
-          }
-          if (wide) {
-            const uint4 v8 = pair8(pk[0], pk[1]);
-            if (m < g.m) {
-              const int f = nt + 8 * q + 8 * hf;  // first of this lane's 8 features
-              uint16_t* dst = E == G_QKV ? (blk ? base + 8 * q + 8 * hf : qkv_dst(g, qkv_feat_at(g, fb, 8 * q + 8 * hf), tok))
-                                         : static_cast<uint16_t*>(g.c) + long(m) * g.n + f;
-              *reinterpret_cast<uint4*>(dst) = v8;
-            }
-          } else if (m < g.m) {
-#pragma unroll
-            for (int r = 0; r < 2; ++r) {
-              const int n = nt + 8 * (q + r) + 4 * hf;
-              if (E == G_QKV) {
-                if (n < g.n) *reinterpret_cast<uint2*>(qkv_dst(g, feat[r], tok)) = make_uint2(pk[r][0], pk[r][1]);
-              } else if (n + 3 < g.n && (g.n & 3) == 0) {
-                *reinterpret_cast<uint2*>(static_cast<uint16_t*>(g.c) + long(m) * g.n + n) =
-                    make_uint2(pk[r][0], pk[r][1]);
-              } else {
-                uint16_t* c = static_cast<uint16_t*>(g.c) + long(m) * g.n + n;
-                const uint32_t w[2] = {pk[r][0], pk[r][1]};
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                  if (n + e < g.n) c[e] = uint16_t(w[e / 2] >> (16 * (e % 2)));
-              }
-            }
-          }
-        }
-      } else {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const f32x4 v = {acc[i][j][4 * q] * rsc[j], acc[i][j][4 * q + 1] * rsc[j], acc[i][j][4 * q + 2] * rsc[j],
-                           acc[i][j][4 * q + 3] * rsc[j]};
-          // store_tile's feature index is nt + 4 * grp: grp = 2q + hf.
-          const QkvFeat feat = E == G_QKV ? qkv_feat_at(g, fb, 8 * q + 4 * hf) : QkvFeat{};
-          store_tile<T, E>(g, v, nt, 2 * q + hf, m, feat, tok);
-        }
-      }
-    }
+    for (int i = 0; i < NBN; ++i)
+      store_block<T, E>(g, acc[i][j], n0 + (TBN / WN) * wn + 32 * i, m, tok, rsc[j], hf);
   }
 }
 
@@ -698,18 +338,20 @@ int launch_gemm_t(const GemmArgs& g, hipStream_t s, const char* what) {
   if (g.m < 1 || g.n < 1 || g.k < 1) return set_error(SFL_ERR_INVALID, "%s: sizes must be positive", what);
   if (g.k % 8) return set_error(SFL_ERR_UNSUPPORTED, "%s: K must be a multiple of 8", what);
   if (g.k % K2 == 0 && long(g.m) * g.k < (1L << 30) && long(g.n) * g.k < (1L << 30)) {
-    const long tiles = long((g.n + TB - 1) / TB) * ((g.m + TB - 1) / TB);
+    Tile16 t = tile16_for(g.m, g.n, g.k, E);
+    if (t <= S128x64 && g.norm_gain && g.norm_part == 128) t = T128x64;
+    if (t <= S128x64) return launch_gemm_small<T, E>(g, t, s, what);
+    const int tn = t == T256x384 || t == T256x256 ? 256 : 128;
+    const int tm = t == T256x384 ? 384 : t == T256x256 ? 256 : t == T128x128 ? 128 : 64;
+    const long tiles = long((g.n + tn - 1) / tn) * ((g.m + tm - 1) / tm);
     if (tiles > (1L << 31) - 1) return set_error(SFL_ERR_UNSUPPORTED, "%s: too many tiles", what);
-    // 256 x 384 tiles where they still give every CU more than one workgroup
-    // (measured against 256 x 256 on the 324M prefill shapes, bit-identical
-    // outputs: q/k/v 437 -> 421 us, output_proj 171 -> 145, w1/w3 640 -> 603,
-    // w2 330 -> 308; 2 x 4 waves of 128 x 96 and a ring of 4 stages of K = 32
-    // were no better).
-    const long big = long((g.n + 255) / 256) * ((g.m + 383) / 384);
-    if (big >= 320)
-      hipLaunchKernelGGL((gemm32_kernel<T, E, 256, 384, 4, 2, 64, 2>), dim3(unsigned(big)), dim3(512), 0, s, g);
-    else
-      hipLaunchKernelGGL((gemm32_kernel<T, E, 128, 128, 2, 2, 64, 2>), dim3(unsigned(tiles)), dim3(kThreads), 0, s, g);
+    const dim3 grid{unsigned(tiles)};
+    switch (t) {
+      case T256x384: hipLaunchKernelGGL((gemm32_kernel<T, E, 256, 384, 4, 2, 64, 2>), grid, dim3(512), 0, s, g); break;
+      case T256x256: hipLaunchKernelGGL((gemm32_kernel<T, E, 256, 256, 4, 2, 64, 2>), grid, dim3(512), 0, s, g); break;
+      case T128x128: hipLaunchKernelGGL((gemm32_kernel<T, E, 128, 128, 2, 2, 64, 2>), grid, dim3(256), 0, s, g); break;
+      default: hipLaunchKernelGGL((gemm32_kernel<T, E, 128, 64, 2, 2, 64, 2>), grid, dim3(256), 0, s, g); break;
+    }
     return check_launch(what);
   }
   dim3 grid((g.n + TN - 1) / TN, (g.m + TM - 1) / TM);
@@ -809,6 +451,45 @@ __global__ __launch_bounds__(256) void norm_scale_kernel(const float* __restrict
 }
 
 }  // namespace
+
+// Which tile a shape runs on. Up to one tile per CU the smallest that still
+// gives every workgroup its own CU wins (K-split tiles, gemm_small.hip), except
+// that 128 x 64 splits K only from K = 1024 on: below, too few chunks per wave
+// repay its reduction (SwiGLU N 2688 K 512 M 512: 7.4 us shared, 8.3 split;
+// residual N 1024 K 2752 M 2048: 31.3 shared, 24.3 split). Beyond, the shapes
+// differ mostly by how their last round of workgroups fills the chip, so the
+// time is estimated from rounds: 128 x 64 runs 3 workgroups per CU, 128 x 128
+// two, the larger ones one, and a round costs (in units of a full round of
+// 128 x 128, 18-33 us at K = 1024 by epilogue) what the tables below hold,
+// measured over N 512..5504, K 512..2752, M 512..49152 with each epilogue.
+// Against the former rule (256 x 384 from 320 such tiles on, else 128 x 128),
+// same outputs: q/k/v N 2304 K 768 M 2048 19.4 -> 16.0 us, SwiGLU N 5504
+// K 1024 M 4096 55.5 -> 45.3, M 4734 62.7 -> 59.3, residual N 1024 K 2752
+// M 16384 110 -> 98; M 49152 unchanged (256 x 384).
+Tile16 tile16_for(long m, long n, long k, int epi) {
+  constexpr long kCus = 256;
+  const auto count = [&](long tn, long tm) { return ((n + tn - 1) / tn) * ((m + tm - 1) / tm); };
+  if (count(32, 32) <= kCus) return S32x32;
+  if (count(64, 32) <= kCus) return S64x32;
+  if (count(64, 64) <= kCus) return S64x64;
+  if (count(128, 64) <= kCus) return k >= 1024 ? S128x64 : T128x64;
+  // Rounds of up to `per` workgroups per CU: whole rounds at part[per - 1]
+  // plus the last one by how many per CU it needs; past 3 rounds the
+  // workgroups no longer run in step and the fraction counts.
+  const auto cost = [&](long tiles, long per, std::initializer_list<double> part) {
+    const double full = part.begin()[per - 1];
+    const long slots = per * kCus, rem = tiles % slots;
+    if (tiles > 3 * slots) return full * (double(tiles) / double(slots) + 0.25);
+    return full * double(tiles / slots) + (rem == 0 ? 0. : part.begin()[(rem - 1) / kCus]);
+  };
+  const double c64 = cost(count(128, 64), 3, {0.58, 0.70, 0.83});
+  const double c128 = cost(count(128, 128), 2, {0.72, 1.0});
+  const double c256 = cost(count(256, 256), 1, {epi == G_QKV ? 1.8 : 1.6});
+  const double c384 = cost(count(256, 384), 1, {epi == G_QKV ? 2.6 : 2.2});
+  const double best = std::min(std::min(c64, c128), std::min(c256, c384));
+  return best == c384 ? T256x384 : best == c256 ? T256x256 : best == c128 ? T128x128 : T128x64;
+}
+
 }  // namespace sfl
 
 using namespace sfl;
@@ -877,12 +558,11 @@ static bool gemm32_path(int m, int n, int k) {
   return k % K2 == 0 && long(m) * k < (1L << 30) && long(n) * k < (1L << 30);
 }
 
-extern "C" int sfl_gemm_qkv_rope_scaled(const void* a_xg, const void* w_qkv, const float* rscale, int m, int seq,
-                                        int d_model, int heads, const float* cos_t, const float* sin_t,
-                                        void* q_out, void* k_cache, void* v_cache, int capacity, int dtype,
-                                        void* stream) {
-  const char* what = "gemm_qkv_rope_scaled";
-  if (!rscale) return set_error(SFL_ERR_INVALID, "%s: null pointer argument", what);
+// q/k/v of a normalized input scaled by rscale[r], or by the ss_parts sums of squares ss.
+static int gemm_qkv_normed(const char* what, const void* a_xg, const void* w_qkv, const float* rscale,
+                           const float* ss, int ss_parts, int m, int seq, int d_model, int heads,
+                           const float* cos_t, const float* sin_t, void* q_out, void* k_cache, void* v_cache,
+                           int capacity, int dtype, void* stream) {
   if (!gemm32_path(m, 3 * d_model, d_model))
     return set_error(SFL_ERR_UNSUPPORTED, "%s: d_model must be a multiple of %d", what, K2);
   if (!a_xg || !w_qkv || !cos_t || !sin_t || !q_out || !k_cache || !v_cache)
@@ -899,29 +579,63 @@ extern "C" int sfl_gemm_qkv_rope_scaled(const void* a_xg, const void* w_qkv, con
   g.q_out = static_cast<uint16_t*>(q_out); g.k_cache = static_cast<uint16_t*>(k_cache);
   g.v_cache = static_cast<uint16_t*>(v_cache);
   g.vec16 = aligned16(q_out) && aligned16(k_cache) && aligned16(v_cache);
-  g.row_scale = rscale;
+  g.row_scale = rscale; g.ss = ss; g.ss_parts = ss_parts;
   return launch_gemm<G_QKV>(g, dtype, static_cast<hipStream_t>(stream), what);
 }
 
-extern "C" int sfl_gemm_swiglu_scaled(const void* a_xg, const void* w13_interleaved, const float* rscale,
-                                      void* h_out, int m, int d_ff, int k, int dtype, void* stream) {
-  const char* what = "gemm_swiglu_scaled";
-  if (!a_xg || !w13_interleaved || !rscale || !h_out)
-    return set_error(SFL_ERR_INVALID, "%s: null pointer argument", what);
+extern "C" int sfl_gemm_qkv_rope_scaled(const void* a_xg, const void* w_qkv, const float* rscale, int m, int seq,
+                                        int d_model, int heads, const float* cos_t, const float* sin_t,
+                                        void* q_out, void* k_cache, void* v_cache, int capacity, int dtype,
+                                        void* stream) {
+  const char* what = "gemm_qkv_rope_scaled";
+  if (!rscale) return set_error(SFL_ERR_INVALID, "%s: null pointer argument", what);
+  return gemm_qkv_normed(what, a_xg, w_qkv, rscale, nullptr, 0, m, seq, d_model, heads, cos_t, sin_t, q_out, k_cache,
+                         v_cache, capacity, dtype, stream);
+}
+
+extern "C" int sfl_gemm_qkv_rope_normed(const void* a_xg, const void* w_qkv, const float* ss_parts, int parts, int m,
+                                        int seq, int d_model, int heads, const float* cos_t, const float* sin_t,
+                                        void* q_out, void* k_cache, void* v_cache, int capacity, int dtype,
+                                        void* stream) {
+  const char* what = "gemm_qkv_rope_normed";
+  if (!ss_parts) return set_error(SFL_ERR_INVALID, "%s: null pointer argument", what);
+  if (parts < 1) return set_error(SFL_ERR_INVALID, "%s: parts must be positive", what);
+  return gemm_qkv_normed(what, a_xg, w_qkv, nullptr, ss_parts, parts, m, seq, d_model, heads, cos_t, sin_t, q_out,
+                         k_cache, v_cache, capacity, dtype, stream);
+}
+
+static int gemm_swiglu_normed(const char* what, const void* a_xg, const void* w13_interleaved, const float* rscale,
+                              const float* ss, int ss_parts, void* h_out, int m, int d_ff, int k, int dtype,
+                              void* stream) {
+  if (!a_xg || !w13_interleaved || !h_out) return set_error(SFL_ERR_INVALID, "%s: null pointer argument", what);
   if (d_ff % 8) return set_error(SFL_ERR_UNSUPPORTED, "%s: d_ff must be a multiple of 8", what);
   if (!gemm32_path(m, 2 * d_ff, k)) return set_error(SFL_ERR_UNSUPPORTED, "%s: K must be a multiple of %d", what, K2);
   GemmArgs g{};
   g.a = static_cast<const uint16_t*>(a_xg); g.w = static_cast<const uint16_t*>(w13_interleaved);
   g.m = m; g.n = 2 * d_ff; g.k = k; g.h_out = static_cast<uint16_t*>(h_out);
   g.vec16 = aligned16(h_out);
-  g.row_scale = rscale;
+  g.row_scale = rscale; g.ss = ss; g.ss_parts = ss_parts;
   return launch_gemm<G_SWIGLU>(g, dtype, static_cast<hipStream_t>(stream), what);
 }
 
-extern "C" int sfl_gemm_residual_norm(const void* a, const void* w, float* x, int m, int n, int k,
-                                      const void* gain_next, void* act_xg, float* ss_parts, int dtype,
-                                      void* stream) {
-  const char* what = "gemm_residual_norm";
+extern "C" int sfl_gemm_swiglu_scaled(const void* a_xg, const void* w13_interleaved, const float* rscale,
+                                      void* h_out, int m, int d_ff, int k, int dtype, void* stream) {
+  const char* what = "gemm_swiglu_scaled";
+  if (!rscale) return set_error(SFL_ERR_INVALID, "%s: null pointer argument", what);
+  return gemm_swiglu_normed(what, a_xg, w13_interleaved, rscale, nullptr, 0, h_out, m, d_ff, k, dtype, stream);
+}
+
+extern "C" int sfl_gemm_swiglu_normed(const void* a_xg, const void* w13_interleaved, const float* ss_parts, int parts,
+                                      void* h_out, int m, int d_ff, int k, int dtype, void* stream) {
+  const char* what = "gemm_swiglu_normed";
+  if (!ss_parts) return set_error(SFL_ERR_INVALID, "%s: null pointer argument", what);
+  if (parts < 1) return set_error(SFL_ERR_INVALID, "%s: parts must be positive", what);
+  return gemm_swiglu_normed(what, a_xg, w13_interleaved, nullptr, ss_parts, parts, h_out, m, d_ff, k, dtype, stream);
+}
+
+static int gemm_residual_norm(const char* what, const void* a, const void* w, float* x, int m, int n, int k,
+                              const void* gain_next, void* act_xg, float* ss_parts, int part, int dtype,
+                              void* stream) {
   if (!a || !w || !x || !gain_next || !act_xg || !ss_parts)
     return set_error(SFL_ERR_INVALID, "%s: null pointer argument", what);
   if (m < 1 || n < 1 || k < 1) return set_error(SFL_ERR_INVALID, "%s: sizes must be positive", what);
@@ -936,8 +650,26 @@ extern "C" int sfl_gemm_residual_norm(const void* a, const void* w, float* x, in
   g.norm_gain = static_cast<const uint16_t*>(gain_next);
   g.norm_act = static_cast<uint16_t*>(act_xg);
   g.norm_ss = ss_parts;
+  g.norm_part = part;
   g.vec16 = aligned16(act_xg) && n % 8 == 0;  // rows of act start 16-byte aligned
   return launch_gemm<G_PLAIN>(g, dtype, static_cast<hipStream_t>(stream), what);
+}
+
+extern "C" int sfl_gemm_residual_norm(const void* a, const void* w, float* x, int m, int n, int k,
+                                      const void* gain_next, void* act_xg, float* ss_parts, int dtype,
+                                      void* stream) {
+  return gemm_residual_norm("gemm_residual_norm", a, w, x, m, n, k, gain_next, act_xg, ss_parts, 128, dtype, stream);
+}
+
+extern "C" int sfl_gemm_norm_part(int m, int n, int k) { return norm_part_of(tile16_for(m, n, k, G_PLAIN)); }
+
+extern "C" int sfl_gemm_residual_norm_parts(const void* a, const void* w, float* x, int m, int n, int k,
+                                            const void* gain_next, void* act_xg, float* ss_parts, int part,
+                                            int dtype, void* stream) {
+  const char* what = "gemm_residual_norm_parts";
+  if (part != 128 && (m < 1 || n < 1 || part != sfl_gemm_norm_part(m, n, k)))
+    return set_error(SFL_ERR_INVALID, "%s: part must be 128 or sfl_gemm_norm_part(m, n, k)", what);
+  return gemm_residual_norm(what, a, w, x, m, n, k, gain_next, act_xg, ss_parts, part, dtype, stream);
 }
 
 extern "C" int sfl_norm_scale(const float* ss_parts, int parts, int m, int d_model, float* rscale, void* stream) {

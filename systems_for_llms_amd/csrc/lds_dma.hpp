@@ -32,4 +32,20 @@ __device__ __forceinline__ unsigned lds_offset(const void* p) {
 // bits 3:0 and 15:14, expcnt 6:4 and lgkmcnt 11:8 left at their maxima).
 constexpr int sfl_vmcnt(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
 
+// Waits until at most `younger` (<= Y) later stages of L loads each are still
+// in flight; the counts are instruction immediates, hence the chain.
+template <int Y, int L>
+__device__ __forceinline__ void wait_younger(int younger) {
+  static_assert(Y * L <= 63, "vmcnt counts to 63");
+  if constexpr (Y > 0) {
+    if (younger >= Y) {
+      __builtin_amdgcn_s_waitcnt(sfl_vmcnt(Y * L));
+      return;
+    }
+    wait_younger<Y - 1, L>(younger);
+  } else {
+    __builtin_amdgcn_s_waitcnt(sfl_vmcnt(0));
+  }
+}
+
 }  // namespace sfl

@@ -324,19 +324,25 @@ class DecodeSession:
              m_rows, d, code, st)
         # Folded norms: a layer's GEMM input is T(x * g) and the GEMM scales its
         # products by 1 / rms(x); the residual GEMM that updates x also writes the
-        # next norm's input and per-128-feature sums of x^2 (one more small kernel
-        # turns them into the scales), so no pass of its own re-reads x.
+        # next norm's input and sums of x^2 over parts of the features, which the
+        # consumer turns into the scales, so no pass of its own re-reads x.
         self.prefill_norm_folded = fold = self._fold_norm(m_rows)
         layers = self.model.layers
         if fold:
-            parts = -(-d // 128)
-            ss = torch.empty((parts, m_rows), device=dev, dtype=torch.float32)
+            # Features per part, after the output projection and after w2.
+            part_o, part_f = (_lib.lib().sfl_gemm_norm_part(m_rows, d, k) for k in (d, f))
+            parts_o, parts_f = -(-d // part_o), -(-d // part_f)
+            ss = torch.empty((max(parts_o, parts_f), m_rows), device=dev, dtype=torch.float32)
             rsc = torch.empty((m_rows,), device=dev, dtype=torch.float32)
             call("sfl_rmsnorm_rows_scaled", x.data_ptr(), layers[0].attn_norm.weight.data_ptr(), act.data_ptr(),
                  rsc.data_ptr(), m_rows, d, code, st)
         for layer, blk in enumerate(layers):
             kc, vc = self.k_cache[layer], self.v_cache[layer]
-            if fold:
+            if fold and layer > 0:
+                call("sfl_gemm_qkv_rope_normed", act.data_ptr(), self.wqkv[layer].data_ptr(), ss.data_ptr(), parts_f,
+                     m_rows, t, d, h, self.cos_fm.data_ptr(), self.sin_fm.data_ptr(), q.data_ptr(), kc.data_ptr(),
+                     vc.data_ptr(), self.cap, code, st)
+            elif fold:
                 call("sfl_gemm_qkv_rope_scaled", act.data_ptr(), self.wqkv[layer].data_ptr(), rsc.data_ptr(), m_rows,
                      t, d, h, self.cos_fm.data_ptr(), self.sin_fm.data_ptr(), q.data_ptr(), kc.data_ptr(),
                      vc.data_ptr(), self.cap, code, st)
@@ -348,11 +354,11 @@ class DecodeSession:
                      self.cap, code, st)
             causal_prefill(q, kc[:, :, :t], vc[:, :, :t], attn.transpose(1, 2))
             if fold:
-                call("sfl_gemm_residual_norm", attn.data_ptr(), blk.attn.output_proj.weight.data_ptr(), x.data_ptr(),
-                     m_rows, d, d, blk.ffn_norm.weight.data_ptr(), act.data_ptr(), ss.data_ptr(), code, st)
-                call("sfl_norm_scale", ss.data_ptr(), parts, m_rows, d, rsc.data_ptr(), st)
-                call("sfl_gemm_swiglu_scaled", act.data_ptr(), w13[layer].data_ptr(), rsc.data_ptr(), hid.data_ptr(),
-                     m_rows, f, d, code, st)
+                call("sfl_gemm_residual_norm_parts", attn.data_ptr(), blk.attn.output_proj.weight.data_ptr(),
+                     x.data_ptr(), m_rows, d, d, blk.ffn_norm.weight.data_ptr(), act.data_ptr(), ss.data_ptr(), part_o,
+                     code, st)
+                call("sfl_gemm_swiglu_normed", act.data_ptr(), w13[layer].data_ptr(), ss.data_ptr(), parts_o,
+                     hid.data_ptr(), m_rows, f, d, code, st)
             else:
                 call("sfl_gemm", attn.data_ptr(), blk.attn.output_proj.weight.data_ptr(), x.data_ptr(),
                      m_rows, d, d, code, F32, 1, st)
@@ -360,9 +366,9 @@ class DecodeSession:
                      code, code, st)
                 call("sfl_gemm_swiglu", act.data_ptr(), w13[layer].data_ptr(), hid.data_ptr(), m_rows, f, d, code, st)
             if fold and layer + 1 < len(layers):
-                call("sfl_gemm_residual_norm", hid.data_ptr(), blk.ffn.w2.weight.data_ptr(), x.data_ptr(), m_rows,
-                     d, f, layers[layer + 1].attn_norm.weight.data_ptr(), act.data_ptr(), ss.data_ptr(), code, st)
-                call("sfl_norm_scale", ss.data_ptr(), parts, m_rows, d, rsc.data_ptr(), st)
+                call("sfl_gemm_residual_norm_parts", hid.data_ptr(), blk.ffn.w2.weight.data_ptr(), x.data_ptr(),
+                     m_rows, d, f, layers[layer + 1].attn_norm.weight.data_ptr(), act.data_ptr(), ss.data_ptr(),
+                     part_f, code, st)
             else:
                 call("sfl_gemm", hid.data_ptr(), blk.ffn.w2.weight.data_ptr(), x.data_ptr(), m_rows, d, f, code, F32,
                      1, st)
