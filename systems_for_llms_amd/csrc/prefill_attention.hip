@@ -134,13 +134,22 @@ __device__ __forceinline__ bool allowed_flat(const MaskArgs& m, int q, int k, in
 // group gained less, 12-16 the same, all 32 at once lost the gain).
 constexpr int kXcds = 8;
 constexpr int kTileOrderHeads = 8;
+constexpr int kXcdCus = 32;
 __device__ __forceinline__ int2 attn_tile(int nqt, int nbh) {
   const int total = nqt * nbh;
   const int blk = int(blockIdx.x);
-  const int x = blk % kXcds, idx = blk / kXcds;
+  const int x = blk % kXcds;
+  int idx = blk / kXcds;
   const int base = total / kXcds, extra = total % kXcds;
   const int start = x * base + min(x, extra);
   const int len = base + (x < extra);
+  // A grid of up to 4 workgroups per CU is all on the chip at once, so nothing
+  // evens the CUs out later: every other round of the XCD's CUs is dealt
+  // backwards, so that with the rows in descending length a CU gets a long row
+  // with a short one (causal 16x16x256 at head dim 32 16.6 -> 14.7 us, 8x12x1024
+  // at head dim 64 1-2% of its 34; larger grids do not gain).
+  const int round0 = idx & ~(kXcdCus - 1);
+  if (len <= 4 * kXcdCus && (idx & kXcdCus)) idx = round0 + min(kXcdCus, len - round0) - 1 - (idx - round0);
   if (len >= 2 * nqt && start % nqt == 0 && len % nqt == 0) {
     constexpr int G = kTileOrderHeads;
     const int heads = len / nqt;
@@ -717,12 +726,13 @@ template <> __device__ __forceinline__ float first_pair<f16_t>(uint32_t pk, uint
 // wave-uniform branch on the scores alone: with two instantiations of the
 // whole tile the compiler kept the O accumulators of one in a second register
 // set and copied them every tile (33 moves, and spills at D = 128).
-template <typename T, int D>
+template <typename T, int D, bool kDocs>
 __device__ __forceinline__ void attn32_tile(const AttnArgs& a, const uint4 (&kt)[BK][D / 8],
                                             const uint4 (&vt)[BK][D / 8], const u32x4 (&qreg)[D / 16],
                                             f32x16 (&oacc)[D / 32], float& m_run, float& l_run, float& m_lim,
                                             float& m_sub, int c, int h, int qrow, int k0, bool full,
-                                            const unsigned (&vlane)[D / 32], bool masked) {
+                                            const unsigned (&vlane)[D / 32], bool masked, int64_t dq,
+                                            const int64_t* dk) {
   const int n = a.n;
   f32x16 sacc[2];
   // S^T for key block kb2 (keys 32 kb2 .. +31 of the tile).
@@ -735,35 +745,60 @@ __device__ __forceinline__ void attn32_tile(const AttnArgs& a, const uint4 (&kt)
       sacc[kb2] = mfma32<T>(u32x4{kr.x, kr.y, kr.z, kr.w}, qreg[ks], sacc[kb2]);
     }
   };
+  // Head dim 128, full tiles: the two blocks' chains alternate, operands read
+  // four ahead (left to itself the compiler runs one chain after the other:
+  // causal 1x8x4096 84 -> 89 us).
+  auto both = [&]() {
+#pragma unroll
+    for (int j = 0; j < 16; ++j) sacc[0][j] = sacc[1][j] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks)
+#pragma unroll
+      for (int kb2 = 0; kb2 < 2; ++kb2) {
+        const uint4 kr = kt[32 * kb2 + c][(D / 16 * h + ks) ^ k_swizzle<D>(c)];
+        sacc[kb2] = mfma32<T>(u32x4{kr.x, kr.y, kr.z, kr.w}, qreg[ks], sacc[kb2]);
+      }
+    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);  // LDS reads
+#pragma unroll
+    for (int i = 4; i < D / 16 * 2; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+  };
   // The scores are computed inside each branch (the masked one takes the
   // blocks in the other order, so the compiler cannot hoist them above the
   // branch): both branches then define the scores afresh, and the join needs
   // no copy of them (with the MFMAs shared ahead of the branch the full-tile
   // path copied all 32 scores every tile).
   if (!masked) {  // wave-uniform: full tiles skip the token mask
-    scores(0);
-    scores(1);
-  } else {
-    scores(1);
-    scores(0);
-    if (!a.m.docs) {
-      const KeyRanges kr = key_ranges(a.m, qrow, n, k0 + 4 * h, full);
-#pragma unroll
-      for (int i = 0; i < 32; ++i) {
-        const int j = i % 16;
-        const int cc = 32 * (i / 16) + 8 * (j / 4) + j % 4;
-        const bool ok = (unsigned(cc + kr.a) <= unsigned(kr.w)) | (cc <= kr.p);
-        sacc[i / 16][j] = ok ? sacc[i / 16][j] : -INFINITY;
-      }
+    if constexpr (D == 128) {
+      both();
     } else {
-      const int64_t dq = a.m.docs[min(qrow, n - 1)];
+      scores(1);
+      scores(0);
+    }
+  } else {
+    scores(0);
+    scores(1);
+    const KeyRanges kr = key_ranges(a.m, qrow, n, k0 + 4 * h, full);
 #pragma unroll
-      for (int i = 0; i < 32; ++i) {
-        const int j = i % 16;
-        const int key = k0 + 32 * (i / 16) + 8 * (j / 4) + 4 * h + j % 4;
-        const int64_t dk = a.m.docs[min(key, n - 1)];
-        const bool ok = full ? (key < n) & (qrow < n) : allowed_flat(a.m, qrow, key, n, dq, dk);
-        sacc[i / 16][j] = ok ? sacc[i / 16][j] : -INFINITY;
+    for (int i = 0; i < 32; ++i) {
+      const int j = i % 16;
+      const int cc = 32 * (i / 16) + 8 * (j / 4) + j % 4;
+      const bool ok = (unsigned(cc + kr.a) <= unsigned(kr.w)) | (cc <= kr.p);
+      sacc[i / 16][j] = ok ? sacc[i / 16][j] : -INFINITY;
+    }
+    if (kDocs && !full) {  // and the query's document (wave-uniform branch)
+#pragma unroll
+      for (int i = 0; i < 32; i += 4) {
+        const int at = 32 * (i / 16) + 8 * (i % 16 / 4) + 4 * h;  // keys k0 + at .. + 3
+        const longlong2 d0 = *reinterpret_cast<const longlong2*>(&dk[at]);
+        const longlong2 d1 = *reinterpret_cast<const longlong2*>(&dk[at + 2]);
+        sacc[i / 16][i % 16] = d0.x == dq ? sacc[i / 16][i % 16] : -INFINITY;
+        sacc[i / 16][i % 16 + 1] = d0.y == dq ? sacc[i / 16][i % 16 + 1] : -INFINITY;
+        sacc[i / 16][i % 16 + 2] = d1.x == dq ? sacc[i / 16][i % 16 + 2] : -INFINITY;
+        sacc[i / 16][i % 16 + 3] = d1.y == dq ? sacc[i / 16][i % 16 + 3] : -INFINITY;
       }
     }
   }
@@ -940,13 +975,17 @@ constexpr int kA32Waves = 4;
 // merge of its two rows' tile lists; a wave skips (but still synchronises on)
 // a tile its own row does not list, so each row processes exactly its own
 // tiles, as the 64-query tiling would.
-// Head dim 64: 32 KB of LDS per workgroup, 168 VGPRs, 3 waves per SIMD. Head
+// Head dim 64: 32 KB of LDS per workgroup and 122 VGPRs (126 with documents), 4
+// waves per SIMD. Documents are an instantiation of their own: their labels in
+// registers had held the others to 146 VGPRs and 3 waves (window 1023 + prefix
+// 256, 4x16x4096: 115 -> 108 us; causal 16x16x3072 393 -> 380). Head
 // dim 128: the same layout with 256-byte rows (64 KB, two workgroups per CU,
 // 2 waves per SIMD), 8 k-steps per score block and 4 dim tiles of O.
-template <int D> constexpr int attn32_waves_per_eu() { return D == 64 ? 3 : 2; }
+template <int D, int NW, bool kDocs>
+constexpr int attn32_waves_per_eu() { return D == 64 && (NW == 4 || !kDocs) ? 3 : 2; }
 
-template <typename T, int D, int NW>
-__global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(attn32_waves_per_eu<D>())))
+template <typename T, int D, int NW, bool kDocs>
+__global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(attn32_waves_per_eu<D, NW, kDocs>())))
 void masked_attention32_kernel(AttnArgs a) {
   static_assert(NW == 2 || NW == 4, "one or two 64-query rows per workgroup");
   constexpr int NR = NW / 2;     // 64-query schedule rows per workgroup
@@ -955,6 +994,7 @@ void masked_attention32_kernel(AttnArgs a) {
   constexpr int RPL = 64 / SL;   // rows one 1 KB load moves
   __shared__ __align__(16) uint4 k_s[2][BK][SL];  // [key][16-byte slot s at s ^ k_swizzle<D>(key)]
   __shared__ __align__(16) uint4 v_s[2][BK][SL];  // [key][16-byte slot, see vt_slot]
+  __shared__ __align__(16) int64_t doc_s[kDocs ? NW * BK : 1];  // the tile's document labels, one copy per wave
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
   const int half = wave / 2;
@@ -1034,19 +1074,33 @@ void masked_attention32_kernel(AttnArgs a) {
                  unsigned(k0_ + RPL * ch_) * vrow_bytes);                                   \
     }                                                                                       \
   }
+  // Document labels: the query's, and lane l's of key l of the next tile,
+  // loaded with the tile and handed round through LDS by the wave that needs
+  // them. (A masked tile that loaded its 32 keys' labels from memory, one load
+  // per score behind the K/V loads in flight, took ~20 us: 2 x 8 x 2999 x 128
+  // with 6 documents 110 -> 54 us.)
+  const int64_t dq = kDocs ? a.m.docs[min(qrow, n - 1)] : 0;
+  int64_t dnext = 0;
   // One key tile: S^T, masked online softmax, O^T += V^T P^T.
   MergedTile cur = next_tile(a, rows);
-  if (cur.kb != INT_MAX) SFL_A32_LOAD(cur.kb, 0)
+  if (cur.kb != INT_MAX) {
+    if constexpr (kDocs) dnext = a.m.docs[min(cur.kb * BK + lane, n - 1)];
+    SFL_A32_LOAD(cur.kb, 0)
+  }
   __builtin_amdgcn_s_waitcnt(sfl_vmcnt(0));
   __syncthreads();
   for (int buf = 0; cur.kb != INT_MAX; buf ^= 1) {
     const MergedTile nxt = next_tile(a, rows);
+    if constexpr (kDocs) {
+      doc_s[wave * BK + lane] = dnext;
+      if (nxt.kb != INT_MAX) dnext = a.m.docs[min(nxt.kb * BK + lane, n - 1)];
+    }
     if (nxt.kb != INT_MAX) SFL_A32_LOAD(nxt.kb, buf ^ 1)
     const int k0 = cur.kb * BK;
     const bool full = (NR == 2 && half ? cur.full[1] : cur.full[0]) && a.s.use_full;
     if (NR == 2 && half ? cur.in[1] : cur.in[0]) {
-      attn32_tile<T, D>(a, k_s[buf], v_s[buf], qreg, oacc, m_run, l_run, m_lim, m_sub, c, h, qrow, k0, full, vlane,
-                        !(full && k0 + BK <= n));
+      attn32_tile<T, D, kDocs>(a, k_s[buf], v_s[buf], qreg, oacc, m_run, l_run, m_lim, m_sub, c, h, qrow, k0, full, vlane,
+                        !(full && k0 + BK <= n), dq, doc_s + (kDocs ? wave * BK : 0));
     }
     __builtin_amdgcn_s_waitcnt(sfl_vmcnt(0));  // the next K and V tiles have landed
     __syncthreads();
@@ -1096,6 +1150,12 @@ inline long row_keys(const MaskArgs& m, long n) {
 #endif
 constexpr long kShortRowKeys = SFL_A32_SHORT_KEYS;
 
+template <typename T, int D, int NW>
+const void* attn32_fn(const MaskArgs& m) {
+  return m.docs ? reinterpret_cast<const void*>(&masked_attention32_kernel<T, D, NW, true>)
+                : reinterpret_cast<const void*>(&masked_attention32_kernel<T, D, NW, false>);
+}
+
 template <typename T>
 MaskedLaunch select_masked(int dim, long n, long k_row_stride, long v_row_stride, const MaskArgs& m) {
   const bool offsets32 = n * k_row_stride * 2 < (1L << 31) && n * v_row_stride * 2 < (1L << 31);
@@ -1106,16 +1166,16 @@ MaskedLaunch select_masked(int dim, long n, long k_row_stride, long v_row_stride
               unsigned(BQ), unsigned(kThreads)};
     case 64:
       if (offsets32 && one_row)
-        return {reinterpret_cast<const void*>(&masked_attention32_kernel<T, 64, 2>),
+        return {attn32_fn<T, 64, 2>(m),
                 "masked_attention32_kernel<D=64, 2 waves>", unsigned(BQ), unsigned(2 * kWave)};
       if (offsets32)
-        return {reinterpret_cast<const void*>(&masked_attention32_kernel<T, 64, kA32Waves>),
+        return {attn32_fn<T, 64, kA32Waves>(m),
                 "masked_attention32_kernel<D=64>", unsigned(2 * BQ), unsigned(kA32Waves * kWave)};
       return {reinterpret_cast<const void*>(&masked_attention_pair_kernel<T>), "masked_attention_pair_kernel<D=64>",
               unsigned(BQ), unsigned(kPairWaves * kWave)};
     case 128:  // (one row per workgroup at D = 128 needs 300 VGPRs: one wave per SIMD)
       if (offsets32)
-        return {reinterpret_cast<const void*>(&masked_attention32_kernel<T, 128, kA32Waves>),
+        return {attn32_fn<T, 128, kA32Waves>(m),
                 "masked_attention32_kernel<D=128>", unsigned(2 * BQ), unsigned(kA32Waves * kWave)};
       return {reinterpret_cast<const void*>(&masked_attention_kernel<T, 128>), "masked_attention_kernel<D=128>",
               unsigned(BQ), unsigned(kThreads)};

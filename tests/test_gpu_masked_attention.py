@@ -70,6 +70,26 @@ def test_document_masks_csr():
     check(q, k, v, MaskSpec(causal=True, same_document=True), torch.tensor(docs), "csr", True)
 
 
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("n", [1, 63, 65, 128, 515])
+def test_document_labels_at_tile_edges(n, d):
+    """Scattered labels that differ in their upper 32 bits only, at the edges of the key tiles."""
+    g = torch.Generator().manual_seed(n)
+    docs = (torch.randint(0, 3, (n,), generator=g) << 32).sort().values
+    docs[n // 2:] = docs[n // 2:][torch.randperm(n - n // 2, generator=g)]
+    q, k, v = inputs(1, 3, n, d, torch.bfloat16, n + d)
+    for spec in (MaskSpec(same_document=True), MaskSpec(causal=True, same_document=True),
+                 MaskSpec(causal=True, window_left=70, same_document=True, global_prefix=5)):
+        check(q, k, v, spec, docs.tolist(), "csr", True)
+
+
+@pytest.mark.parametrize("b,h,n,d", [(5, 12, 1000, 64), (3, 11, 600, 32), (9, 15, 300, 128)])
+def test_every_query_tile_is_dealt_once(b, h, n, d):
+    """Grids of one to four workgroups per CU, the last round of an XCD partial."""
+    q, k, v = inputs(b, h, n, d, torch.float16, n)
+    check(q, k, v, MaskSpec(causal=True), None, "interval", True)
+
+
 def test_schedule_compiled_for_other_tiles_is_recompiled():
     q, k, v = inputs(1, 2, 300, 64, torch.bfloat16, 3)
     for block in (16, 32, 128):
