@@ -3,12 +3,15 @@
 //
 // The reference's float32 TransformerLM.forward (src/llmlab/model/
 // transformer.py:121-139) runs every Linear (layers.py:34-35) and the
-// attention (attention.py:61-98,187-197) in fp32; these kernels keep every
-// product and sum in fp32, so they differ from it only by the order of fp32
-// additions.
+// attention (attention.py:61-98,187-197) in fp32; these kernels form every
+// product of fp32 values to at least fp32 accuracy and sum in fp32, so they
+// differ from it by the order of fp32 additions.
 //
-// GEMM: C^T[n][m] = sum_k W[n][k] A[m][k] on v_mfma_f32_32x32x2_f32 (fp32
-// operands, fp32 accumulation). A workgroup of 4 waves (2 x 2) computes 64
+// GEMM: K a multiple of 32 and operands under 2 GiB run gemm_split_kernel
+// (gemm_split.hpp: K split over the waves, each fp32 product formed exactly
+// from bf16 pieces on the bf16 matrix cores). Other shapes run
+// gemm_f32_kernel: C^T[n][m] = sum_k W[n][k] A[m][k] on v_mfma_f32_32x32x2_f32
+// (fp32 operands, fp32 accumulation). A workgroup of 4 waves (2 x 2) computes 64
 // features x 64 tokens, a wave one 32 x 32 block; K advances by 32 through two
 // LDS stages (rows padded to 36 floats), the next stage's global loads in
 // registers while the current one computes. A lane reads 16 bytes -- 4
@@ -26,12 +29,10 @@
 // exact fp32 online softmax (base 2, the scale folded into q).
 #include <math.h>
 
-#include "gemm_f32.hpp"
+#include "gemm_split.hpp"
 
 namespace sfl {
 namespace {
-
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int FT = 64;        // features and tokens per workgroup
 constexpr int FK = 32;        // K per LDS stage
@@ -41,9 +42,6 @@ constexpr int kF32Threads = 256;
 __device__ __forceinline__ f32x16 mfma32f(float a, float b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
-
-// silu(a) * c with an IEEE exponential (layers.py:102-104,114-115).
-__device__ __forceinline__ float silu_mul_f32(float a, float c) { return a / (1.f + expf(-a)) * c; }
 
 template <int E>
 __global__ __launch_bounds__(kF32Threads) void gemm_f32_kernel(F32GemmArgs g) {
@@ -109,66 +107,7 @@ __global__ __launch_bounds__(kF32Threads) void gemm_f32_kernel(F32GemmArgs g) {
 #undef SFL_F32_GLOAD
 #undef SFL_F32_SSTORE
 
-  // acc[4q + e] holds feature n0 + 32 wn + 8q + 4hf + e of token m0 + 32 wm + l32.
-  const int m = m0 + 32 * wm + l32;
-  if (m >= g.m) return;
-  const int nt = n0 + 32 * wn;
-  if constexpr (E == F32_SWIGLU) {
-    // Groups q = 0, 2 are W1 rows, q + 1 the W3 rows of the same hidden features
-    // nt/2 + 4q + 4hf .. +3.
-#pragma unroll
-    for (int q = 0; q < 4; q += 2) {
-      const int f = nt / 2 + 4 * q + 4 * hf;
-      if (f >= g.n / 2) continue;
-      float h[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) h[e] = silu_mul_f32(acc[4 * q + e], acc[4 * q + 4 + e]);
-      *reinterpret_cast<float4*>(g.h_out + long(m) * (g.n / 2) + f) = make_float4(h[0], h[1], h[2], h[3]);
-    }
-  } else if constexpr (E == F32_QKV) {
-    const int b = m / g.seq, t = m - (m / g.seq) * g.seq;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int n = nt + 8 * q + 4 * hf;
-      if (n >= g.n) continue;
-      const int section = n / g.d_model;
-      const int fi = n - section * g.d_model;
-      const int head = fi / g.head_dim, dim = fi - (fi / g.head_dim) * g.head_dim;
-      float y[4] = {acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
-      if (section < 2) {  // RoPE pairs (dim, dim+1), (dim+2, dim+3) (attention.py:44-58)
-        const long r0 = long(dim / 2) * g.cap + t;
-        const float c0 = g.cos_t[r0], c1 = g.cos_t[r0 + g.cap];
-        const float s0 = g.sin_t[r0], s1 = g.sin_t[r0 + g.cap];
-        const float e0 = y[0], o0 = y[1], e1 = y[2], o1 = y[3];
-        y[0] = e0 * c0 - o0 * s0;
-        y[1] = e0 * s0 + o0 * c0;
-        y[2] = e1 * c1 - o1 * s1;
-        y[3] = e1 * s1 + o1 * c1;
-      }
-      float* dst = section == 0 ? g.q_out + ((long(b) * g.heads + head) * g.seq + t) * g.head_dim + dim
-                                : (section == 1 ? g.k_cache : g.v_cache) +
-                                      ((long(b) * g.heads + head) * g.cap + t) * g.head_dim + dim;
-      *reinterpret_cast<float4*>(dst) = make_float4(y[0], y[1], y[2], y[3]);
-    }
-  } else {  // F32_PLAIN
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int n = nt + 8 * q + 4 * hf;
-      float* c = g.c + long(m) * g.n + n;
-      if (n + 3 < g.n && (g.n & 3) == 0) {
-        float4 v = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
-        if (g.accumulate) {
-          const float4 old = *reinterpret_cast<const float4*>(c);
-          v = make_float4(old.x + v.x, old.y + v.y, old.z + v.z, old.w + v.w);
-        }
-        *reinterpret_cast<float4*>(c) = v;
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (n + e < g.n) c[e] = (g.accumulate ? c[e] : 0.f) + acc[4 * q + e];
-      }
-    }
-  }
+  store_block_f32<E>(g, acc, n0 + 32 * wn, m0 + 32 * wm + l32, hf);
 }
 
 struct F32AttnArgs {
@@ -243,6 +182,37 @@ __global__ __launch_bounds__(kF32Threads) void causal_attention_f32_kernel(F32At
     *reinterpret_cast<float4*>(op + d) = make_float4(o[d] * inv, o[d + 1] * inv, o[d + 2] * inv, o[d + 3] * inv);
 }
 
+template <int E, int TBN, int TBM, int KS, int NW, int NS>
+int launch_tile(const F32GemmArgs& g, hipStream_t s, const char* what) {
+  const long tiles = long((g.n + TBN - 1) / TBN) * ((g.m + TBM - 1) / TBM);
+  if (tiles > (1L << 31) - 1) return set_error(SFL_ERR_UNSUPPORTED, "%s: too many tiles", what);
+  hipLaunchKernelGGL((gemm_split_kernel<float, E, TBN, TBM, KS, NW, NS>), dim3(unsigned(tiles)), dim3(NW * kWave), 0,
+                     s, g);
+  return check_launch(what);
+}
+
+// Tile of an fp32 GEMM. 32 x 32 runs two workgroups per CU, and while that
+// covers the grid no larger tile is faster; 64 x 64 on 8 waves fills a CU
+// alone; beyond, 64 x 64 (two per CU) or 64 x 32 (three), whichever leaves the
+// fullest CU less to do (a 64 x 32 tile costs 1.12 halves of a 64 x 64 one).
+// us, gemm_f32_kernel -> this: M 1000 N 512 K 512 19.6 -> 8.8 (32 x 32);
+// M 2048 N 512 K 1344 63 -> 22 (64 x 64, 8 waves); M 1000 N 2304 K 768
+// 57 -> 33 (64 x 32; 64 x 64 34); M 4000 N 2304 K 768 162 -> 95, M 12000 N 4096
+// K 768 749 -> 483 (64 x 64: 156 TFLOP/s). 128 x 64 and 128 x 128 gain only at
+// K = 2752 (7-11%).
+template <int E>
+int launch_split(const F32GemmArgs& g, hipStream_t s, const char* what) {
+  constexpr long kCus = 256;
+  const auto count = [&](long tn, long tm) { return ((g.n + tn - 1) / tn) * ((g.m + tm - 1) / tm); };
+  if (count(32, 32) <= 2 * kCus) return launch_tile<E, 32, 32, 32, 4, 2>(g, s, what);
+  const long t64 = count(64, 64);
+  if (t64 <= kCus) return launch_tile<E, 64, 64, 16, 8, 1>(g, s, what);
+  const double most64 = 2. * double((t64 + kCus - 1) / kCus);
+  const double most32 = 1.12 * double((count(64, 32) + kCus - 1) / kCus);
+  if (most32 < most64) return launch_tile<E, 64, 32, 16, 4, 2>(g, s, what);
+  return launch_tile<E, 64, 64, 16, 4, 2>(g, s, what);
+}
+
 }  // namespace
 
 int launch_gemm_f32(const F32GemmArgs& g, int epi, hipStream_t stream, const char* what) {
@@ -251,6 +221,14 @@ int launch_gemm_f32(const F32GemmArgs& g, int epi, hipStream_t stream, const cha
   const auto a16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   if (!a16(g.a) || !a16(g.w))
     return set_error(SFL_ERR_INVALID, "%s: fp32 operands must be 16-byte aligned", what);
+  // 32-bit byte offsets and whole 128-byte K chunks: the split kernel.
+  if (g.k % 32 == 0 && long(g.m) * g.k < (1L << 29) && long(g.n) * g.k < (1L << 29)) {
+    switch (epi) {
+      case F32_QKV: return launch_split<F32_QKV>(g, stream, what);
+      case F32_SWIGLU: return launch_split<F32_SWIGLU>(g, stream, what);
+      default: return launch_split<F32_PLAIN>(g, stream, what);
+    }
+  }
   const dim3 grid(unsigned((g.n + FT - 1) / FT), unsigned((g.m + FT - 1) / FT));
   if (grid.y > 65535) return set_error(SFL_ERR_UNSUPPORTED, "%s: M too large", what);
   switch (epi) {
