@@ -78,4 +78,45 @@ typedef __attribute__((address_space(3))) i16x4_t lds_i16x4_t;
 
 constexpr float kLazyMax = 8.f;
 
+// Workgroup -> (query tile, batch * head) of a 1-D grid, XCD-aware. Workgroups
+// are dealt to the 8 XCDs round-robin and each XCD has its own 4 MB L2, so XCD
+// x takes a contiguous range of the head-major tile order: the ~100
+// workgroups an XCD runs at once then share the K/V of 2-3 heads (0.8 MB per
+// head at 3072 x 64 bf16) instead of every XCD streaming every head's K/V.
+// Query tiles run last-first, so the longest causal rows start first. When
+// the XCD's range is two or more whole heads, it is dealt query-tile major
+// across groups of up to kTileOrderHeads heads: the tail of each group (and
+// of the range) is then the short rows of several heads, not one head's
+// short rows after other heads' long ones, while the heads an XCD runs at
+// once stay few enough to share their K/V in its L2 (measured: causal
+// 16x16x3072 417 -> 392 us, config 5 125 -> 119 us; 4 or 6 heads per
+// group gained less, 12-16 the same, all 32 at once lost the gain).
+constexpr int kXcds = 8;
+constexpr int kTileOrderHeads = 8;
+constexpr int kXcdCus = 32;
+__device__ __forceinline__ int2 attn_tile(int nqt, int nbh) {
+  const int total = nqt * nbh;
+  const int blk = int(blockIdx.x);
+  const int x = blk % kXcds;
+  int idx = blk / kXcds;
+  const int base = total / kXcds, extra = total % kXcds;
+  const int start = x * base + min(x, extra);
+  const int len = base + (x < extra);
+  // A grid of up to 4 workgroups per CU is all on the chip at once, so nothing
+  // evens the CUs out later: every other round of the XCD's CUs is dealt
+  // backwards, so that with the rows in descending length a CU gets a long row
+  // with a short one (causal 16x16x256 at head dim 32 16.6 -> 14.7 us, 8x12x1024
+  // at head dim 64 1-2% of its 34; larger grids do not gain).
+  const int round0 = idx & ~(kXcdCus - 1);
+  if (len <= 4 * kXcdCus && (idx & kXcdCus)) idx = round0 + min(kXcdCus, len - round0) - 1 - (idx - round0);
+  if (len >= 2 * nqt && start % nqt == 0 && len % nqt == 0) {
+    constexpr int G = kTileOrderHeads;
+    const int heads = len / nqt;
+    const int grp = idx / (G * nqt), g = min(G, heads - grp * G), r = idx - grp * G * nqt;
+    return make_int2(nqt - 1 - r / g, start / nqt + grp * G + r % g);
+  }
+  const int t = start + idx;
+  return make_int2(nqt - 1 - t % nqt, t / nqt);
+}
+
 }  // namespace sfl

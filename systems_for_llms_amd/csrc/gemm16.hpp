@@ -236,7 +236,6 @@ __device__ __forceinline__ int stage_swizzle(int r) {
 // XCD runs at once then cover about 4 token tiles x 8 feature tiles, whose
 // operands stay in (or near) its 4 MB L2 (for 256 x 384 tiles, 448 KB of the
 // 2.5 MB a K step requests are distinct).
-constexpr int kXcds = 8;
 constexpr int kGroupM = 4;
 
 __device__ __forceinline__ int2 xcd_tile(int b, int tn, int tm, int gm = kGroupM) {

@@ -22,11 +22,9 @@
 // a lane, so the epilogues of the 16-bit GEMMs carry over: RoPE pairs in-lane,
 // W1/W3 interleaved in blocks of 8 rows paired in-lane, 16-byte stores.
 //
-// Attention: one workgroup of 256 threads per 64 queries of one (batch, head);
-// four threads per query, each holding a quarter of the head dim of q and of
-// the output. Key/value tiles of 32 rows are staged in LDS; for each key the
-// four threads add their partial dot products with two shuffles and update an
-// exact fp32 online softmax (base 2, the scale folded into q).
+// Attention: one workgroup of 4 waves per 64 queries of one (batch, head), the
+// same pieces on the matrix cores, an exact fp32 online softmax (base 2, the
+// scale folded into q).
 #include <math.h>
 
 #include "gemm_split.hpp"
@@ -119,17 +117,17 @@ struct F32AttnArgs {
 };
 
 constexpr int kAttnQ = 64;   // queries per workgroup
-constexpr int kAttnK = 32;   // keys per LDS tile
+constexpr int kAttnK = 64;   // keys per staged tile
+constexpr int kValuK = 32;   // keys per tile of causal_rows_valu
 
+// The 64 query rows from qb * 64 of one (batch, head) on the VALU: four
+// threads per query, each with a quarter of the head dim; a key above a
+// query's row is never read by it. smem: 2 * kValuK * D floats.
 template <int D>
-__global__ __launch_bounds__(kF32Threads) void causal_attention_f32_kernel(F32AttnArgs a) {
+__device__ __forceinline__ void causal_rows_valu(const F32AttnArgs& a, int qb, int b, int h, float* smem) {
   constexpr int DQ = D / 4;  // head-dim quarter of a thread
-  __shared__ __align__(16) float kt[kAttnK][D];
-  __shared__ __align__(16) float vt[kAttnK][D];
-  const int nqb = (a.n + kAttnQ - 1) / kAttnQ;
-  const int qb = nqb - 1 - int(blockIdx.x % nqb);  // longest rows first
-  const int bh = int(blockIdx.x / nqb);
-  const int b = bh / a.heads, h = bh % a.heads;
+  float (*kt)[D] = reinterpret_cast<float (*)[D]>(smem);
+  float (*vt)[D] = kt + kValuK;
   const int tid = threadIdx.x;
   const int qrow = qb * kAttnQ + tid / 4, part = tid % 4;
   const float* qp = a.q + b * a.qs[0] + h * a.qs[1] + long(min(qrow, a.n - 1)) * a.qs[2] + part * DQ;
@@ -143,16 +141,16 @@ __global__ __launch_bounds__(kF32Threads) void causal_attention_f32_kernel(F32At
   const int kend = min(a.n, qb * kAttnQ + kAttnQ);  // keys 0 .. kend-1 cover every row of the block
   const float* kb = a.k + b * a.ks[0] + h * a.ks[1];
   const float* vb = a.v + b * a.vs[0] + h * a.vs[1];
-  for (int k0 = 0; k0 < kend; k0 += kAttnK) {
+  for (int k0 = 0; k0 < kend; k0 += kValuK) {
     __syncthreads();
-    for (int idx = tid; idx < kAttnK * D / 4; idx += kF32Threads) {
+    for (int idx = tid; idx < kValuK * D / 4; idx += kF32Threads) {
       const int r = idx / (D / 4), c4 = idx % (D / 4);
       const long key = min(k0 + r, a.n - 1);
       *reinterpret_cast<float4*>(&kt[r][4 * c4]) = *reinterpret_cast<const float4*>(kb + key * a.ks[2] + 4 * c4);
       *reinterpret_cast<float4*>(&vt[r][4 * c4]) = *reinterpret_cast<const float4*>(vb + key * a.vs[2] + 4 * c4);
     }
     __syncthreads();
-    const int jn = min(kAttnK, kend - k0);  // uniform over the workgroup
+    const int jn = min(kValuK, kend - k0);  // uniform over the workgroup
     for (int j = 0; j < jn; ++j) {
       float s = 0.f;
 #pragma unroll
@@ -180,6 +178,206 @@ __global__ __launch_bounds__(kF32Threads) void causal_attention_f32_kernel(F32At
 #pragma unroll
   for (int d = 0; d < DQ; d += 4)
     *reinterpret_cast<float4*>(op + d) = make_float4(o[d] * inv, o[d + 1] * inv, o[d + 2] * inv, o[d + 3] * inv);
+}
+
+// Causal attention of 64 queries per workgroup on the bf16 matrix cores, every
+// fp32 operand as three exact bf16 pieces (split3), six products each: S^T =
+// K Q^T and O^T += V^T P^T with the layouts of the 16-bit masked attention
+// (k_swizzle, vt_slot, transpose reads), K and V split once per tile into
+// three LDS planes. Waves 0 and 1 take the first 32 keys of each 64-key tile
+// for queries 0..31 and 32..63, waves 2 and 3 the other 32 keys: a wave's
+// chain -- the longest row bounds a short launch -- is half as long, and the
+// two halves of a row merge through LDS at the end. The softmax is fp32, the
+// row sum over the fp32 probabilities. Against the VALU kernel this replaces
+// (one key at a time, 21 TFLOP/s), causal us: 4x12x1000 D 64 276 -> 58,
+// 2x16x4096 D 64 2215 -> 440, 8x16x256 D 32 53 -> 13, 2x4x2048 D 128
+// 760 -> 145; relative error to float64 3.3e-7 -> 2.5e-7, 5.7e-7 -> 3.4e-7,
+// 2.0e-7 -> 1.6e-7, 4.4e-7 -> 3.3e-7. Bound by the split and softmax VALU work
+// beside ~1500 MFMA cycles per 32 x 32 block at D 64; 3 waves per SIMD there
+// spill (50 registers). A row that comes out NaN (an infinity or NaN
+// in q, k or v, which the pieces do not carry, or which a masked key's zero
+// probability would multiply) sends its workgroup to causal_rows_valu.
+template <int D>
+__global__ __launch_bounds__(kF32Threads) __attribute__((amdgpu_waves_per_eu(D < 64 ? 3 : D == 64 ? 2 : 1)))
+void causal_attention_f32_kernel(F32AttnArgs a) {
+  constexpr int DL = D < 64 ? 64 : D;          // LDS row width (values)
+  constexpr int RS = DL / 8;                   // 16-byte slots per LDS row
+  constexpr int SL = D / 8;                    // of which used
+  constexpr int KS = D / 16;                   // MFMA steps over the head dim
+  constexpr int DT = D < 32 ? 1 : D / 32;      // 32-wide dim tiles of O^T
+  constexpr int NLD = (kAttnK * SL + kF32Threads - 1) / kF32Threads;  // slots a thread stages per operand
+  struct Lds {
+    uint4 k[3][kAttnK][RS];
+    uint4 v[3][kAttnK][RS];
+  };
+  __shared__ __align__(16) Lds st;
+  static_assert(sizeof(Lds) >= sizeof(float) * 2 * kValuK * D, "the VALU rows fit");
+  static_assert(sizeof(Lds) >= sizeof(float) * 2 * kWave * (16 * DT + 2), "the merge rows fit");
+  const int2 tile = attn_tile((a.n + kAttnQ - 1) / kAttnQ, a.batch * a.heads);
+  const int qb = __builtin_amdgcn_readfirstlane(tile.x), bh = __builtin_amdgcn_readfirstlane(tile.y);
+  const int b = bh / a.heads, hd = bh % a.heads;
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int qsub = wave & 1, grp = wave >> 1;  // 32-query half, 32-key half of each tile
+  const int c = lane % 32, h = lane / 32;
+  const int qrow = qb * kAttnQ + 32 * qsub + c;
+
+  // Q^T operand pieces of step ks: dims (D/2) h + 8 ks .. +7, scaled.
+  u32x4 qreg[KS][3];
+  {
+    const float* qp = a.q + b * a.qs[0] + hd * a.qs[1] + long(min(qrow, a.n - 1)) * a.qs[2] + (D / 2) * h;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      uint32_t x[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = __float_as_uint(qp[8 * ks + e] * a.scale_log2);
+      split3(make_uint4(x[0], x[1], x[2], x[3]), make_uint4(x[4], x[5], x[6], x[7]), qreg[ks]);
+    }
+  }
+  const float* kb = a.k + b * a.ks[0] + hd * a.ks[1];
+  const float* vb = a.v + b * a.vs[0] + hd * a.vs[1];
+  uint4 kr[NLD][2], vr[NLD][2];
+  auto load = [&](int t) {
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) {
+      const int idx = min(tid + i * kF32Threads, kAttnK * SL - 1);
+      const long key = min(t * kAttnK + idx / SL, a.n - 1);
+      const float* kp = kb + key * a.ks[2] + 8 * (idx % SL);
+      const float* vp = vb + key * a.vs[2] + 8 * (idx % SL);
+      kr[i][0] = load16(kp);
+      kr[i][1] = load16(kp + 4);
+      vr[i][0] = load16(vp);
+      vr[i][1] = load16(vp + 4);
+    }
+  };
+  unsigned vlane[DT];
+#pragma unroll
+  for (int t = 0; t < DT; ++t) vlane[t] = vt_lane_offset<DL>(lane, t) + unsigned(grp) * 32u * 2u * DL;
+
+  float m_run = -INFINITY, l_run = 0.f;
+  f32x16 o[DT];
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) o[t][j] = 0.f;
+  load(0);
+  for (int t = 0; t <= qb; ++t) {
+    __syncthreads();  // the previous tile is no longer read
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) {
+      const int idx = tid + i * kF32Threads;
+      if (kAttnK * SL % kF32Threads == 0 || idx < kAttnK * SL) {
+        const int r = idx / SL, s = idx % SL;
+        u32x4 pk[3], pv[3];
+        split3(kr[i][0], kr[i][1], pk);
+        split3(vr[i][0], vr[i][1], pv);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+          st.k[p][r][s ^ k_swizzle<DL>(r)] = make_uint4(pk[p][0], pk[p][1], pk[p][2], pk[p][3]);
+          st.v[p][r][vt_slot(s, r)] = make_uint4(pv[p][0], pv[p][1], pv[p][2], pv[p][3]);
+        }
+      }
+    }
+    __syncthreads();
+    if (t < qb) load(t + 1);
+    if (t == qb && grp > qsub) continue;  // keys above every query of the wave
+    constexpr int pa[6] = {2, 1, 0, 1, 0, 0}, pb[6] = {0, 1, 2, 0, 1, 0};  // smallest products first
+    f32x16 s;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) s[j] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      u32x4 kp[3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+        const uint4 r = st.k[p][32 * grp + c][(KS * h + ks) ^ k_swizzle<DL>(c)];
+        kp[p] = u32x4{r.x, r.y, r.z, r.w};
+      }
+#pragma unroll
+      for (int p = 0; p < 6; ++p) s = mfma32<bf16_t>(kp[pa[p]], qreg[ks][pb[p]], s);
+    }
+    if (t == qb && grp == qsub) {  // the diagonal block (attention.py:187-197)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) s[j] = 8 * (j / 4) + 4 * h + j % 4 <= c ? s[j] : -INFINITY;
+    }
+    float mx = s[0];
+#pragma unroll
+    for (int j = 1; j < 16; ++j) mx = fmaxf(mx, s[j]);
+    mx = fmaxf(mx, lane_xor(mx, 32));
+    const float m_new = fmaxf(m_run, mx);
+    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+    m_run = m_new;
+    float sum = 0.f;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      s[j] = __builtin_amdgcn_exp2f(s[j] - m_new);
+      sum += s[j];
+    }
+    l_run = l_run * alpha + sum;
+    if (__ballot(alpha != 1.f)) {
+#pragma unroll
+      for (int d = 0; d < DT; ++d) o[d] *= alpha;
+    }
+#pragma unroll
+    for (int s2 = 0; s2 < 2; ++s2) {
+      uint32_t x[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = __float_as_uint(s[8 * s2 + e]);
+      u32x4 pp[3];
+      split3(make_uint4(x[0], x[1], x[2], x[3]), make_uint4(x[4], x[5], x[6], x[7]), pp);
+#pragma unroll
+      for (int d = 0; d < DT; ++d) {
+        u32x4 vp[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+          const unsigned off = lds_offset(&st.v[p][0][0]) + vlane[d] + 32u * DL * s2;
+          const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(size_t)(off));
+          const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(size_t)(off + 16u * DL));
+          const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
+          vp[p] = u32x4{l2.x, l2.y, h2.x, h2.y};
+        }
+#pragma unroll
+        for (int p = 0; p < 6; ++p) o[d] = mfma32<bf16_t>(vp[pa[p]], pp[pb[p]], o[d]);
+      }
+    }
+  }
+
+  // Waves 2 and 3 hand their half of each row to waves 0 and 1.
+  l_run += lane_xor(l_run, 32);
+  float* const red = reinterpret_cast<float*>(&st) + (qsub * (16 * DT + 2)) * kWave + lane;
+  __syncthreads();
+  if (grp == 1) {
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) red[(16 * d + j) * kWave] = o[d][j];
+    red[16 * DT * kWave] = m_run;
+    red[(16 * DT + 1) * kWave] = l_run;
+  }
+  __syncthreads();
+  bool nan = false;
+  if (grp == 0) {
+    const float m1 = red[16 * DT * kWave], l1 = red[(16 * DT + 1) * kWave];
+    const float top = fmaxf(m_run, m1);
+    const float w0 = __builtin_amdgcn_exp2f(m_run - top), w1 = __builtin_amdgcn_exp2f(m1 - top);
+    const float inv = 1.f / (l_run * w0 + l1 * w1);  // key 0 is always admissible: the sum is at least 1
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        o[d][j] = (o[d][j] * w0 + red[(16 * d + j) * kWave] * w1) * inv;
+        if (D >= 32 || j < 8) nan |= o[d][j] != o[d][j];
+      }
+  }
+  if (__syncthreads_or(nan && qrow < a.n)) return causal_rows_valu<D>(a, qb, b, hd, reinterpret_cast<float*>(&st));
+  if (grp == 1 || qrow >= a.n) return;
+  float* op = a.o + b * a.os[0] + hd * a.os[1] + long(qrow) * a.os[2];
+#pragma unroll
+  for (int d = 0; d < DT; ++d)
+#pragma unroll
+    for (int q = 0; q < (D < 32 ? 2 : 4); ++q)
+      *reinterpret_cast<float4*>(op + 32 * d + 8 * q + 4 * h) =
+          make_float4(o[d][4 * q], o[d][4 * q + 1], o[d][4 * q + 2], o[d][4 * q + 3]);
 }
 
 template <int E, int TBN, int TBM, int KS, int NW, int NS>
