@@ -399,6 +399,39 @@ int sfl_gemm_qkv_rope_normed(const void* a_xg, const void* w_qkv, const float* s
 int sfl_gemm_swiglu_normed(const void* a_xg, const void* w13_interleaved, const float* ss_parts, int parts,
                            void* h_out, int m, int d_ff, int k, int dtype, void* stream);
 
+/* ---- every layer of a prefill in one call ------------------------------------
+ *
+ * Launches, in order, sfl_embed_rows and each layer's sequence of the entry
+ * points above: with fold (16-bit models only, d_model and d_ff multiples of
+ * 64) the folded-norm ones, else sfl_rmsnorm_rows and the unscaled GEMMs; the
+ * attention is causal (sfl_masked_attention on its interval schedule, fp32:
+ * sfl_causal_attention_f32). x holds the last layer's output afterwards. The
+ * pointer arrays are host arrays of one device pointer per layer; buffers as
+ * the entry points describe them, in the model dtype unless typed. ss
+ * [max(ceil(d_model / part))][m] (fold; parts of sfl_gemm_norm_part) and
+ * rscale [m] (fold) are scratch, m = batch * seq. */
+typedef struct {
+  int dtype, layers, batch, seq, d_model, heads, d_ff, capacity, fold;
+  float scale;                    /* attention: head_dim ^ -0.5 */
+  const int64_t* ids;             /* [m] */
+  const void* emb;                /* [vocab, d_model] */
+  const void* const* attn_norm;   /* [d_model] */
+  const void* const* w_qkv;       /* [3 d_model, d_model] */
+  const void* const* w_out;       /* [d_model, d_model] */
+  const void* const* ffn_norm;    /* [d_model] */
+  const void* const* w13;         /* interleaved [2 d_ff, d_model] */
+  const void* const* w2;          /* [d_model, d_ff] */
+  void* const* k_cache;           /* [B, H, capacity, dk] */
+  void* const* v_cache;
+  const float* cos_t;             /* feature-major [dk / 2, capacity] */
+  const float* sin_t;
+  float* x;                       /* [m, d_model] */
+  void *act, *q, *attn, *hidden;  /* [m, d_model], [B, H, T, dk], [B, T, H, dk], [m, d_ff] */
+  float *ss, *rscale;
+} sfl_prefill_args;
+
+int sfl_prefill_layers(const sfl_prefill_args* args, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -56,11 +56,22 @@ SIGNATURES: dict[str, list] = {
     "sfl_gemm_swiglu_scaled": [P, P, P, P, c_int, c_int, c_int, c_int, P],
     "sfl_gemm_qkv_rope_normed": [P, P, P, c_int, c_int, c_int, c_int, c_int, P, P, P, P, P, c_int, c_int, P],
     "sfl_gemm_swiglu_normed": [P, P, P, c_int, P, c_int, c_int, c_int, c_int, P],
+    "sfl_prefill_layers": [P, P],
     "sfl_causal_attention_f32": [P, P, P, P, c_int, c_int, c_int, c_int, POINTER(c_long), POINTER(c_long),
                                  POINTER(c_long), POINTER(c_long), c_float, P],
 }
 
 _LIB = None
+
+
+class PrefillArgs(ctypes.Structure):
+    """``sfl_prefill_args`` of ``include/sfl.h``."""
+
+    _fields_ = ([(n, c_int) for n in ("dtype", "layers", "batch", "seq", "d_model", "heads", "d_ff", "capacity", "fold")]
+                + [("scale", c_float), ("ids", P), ("emb", P)]
+                + [(n, POINTER(P)) for n in ("attn_norm", "w_qkv", "w_out", "ffn_norm", "w13", "w2", "k_cache",
+                                             "v_cache")]
+                + [(n, P) for n in ("cos_t", "sin_t", "x", "act", "q", "attn", "hidden", "ss", "rscale")])
 
 
 class KernelInfo(ctypes.Structure):
@@ -138,6 +149,11 @@ def library_sha256() -> str:
 
         _LIB_SHA256 = hashlib.sha256(LIB_PATH.read_bytes()).hexdigest()
     return _LIB_SHA256
+
+
+def pointers(tensors):
+    """A host array of the tensors' device pointers (they must outlive its use)."""
+    return (P * len(tensors))(*[t.data_ptr() for t in tensors])
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

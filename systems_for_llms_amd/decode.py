@@ -27,7 +27,7 @@ from dataclasses import dataclass
 import torch
 
 from . import _lib
-from . import ops  # noqa: F401  (registers torch.ops.sfl)
+from . import ops  # registers torch.ops.sfl
 
 SUPPORTED_DIMS = (16, 32, 64, 128)
 SUPPORTED_GROUPS = (1, 2, 4, 8)
@@ -111,9 +111,13 @@ class PreparedDecode:
     variant: str
 
     def __call__(self) -> torch.Tensor:
-        torch.ops.sfl.decode_attention(self.q, self.k, self.v, self.lengths, self.partial_max,
-                                       self.partial_sum, self.partial_output, self.output, self.splits,
-                                       self.scale)
+        args = (self.q, self.k, self.v, self.lengths, self.partial_max, self.partial_sum, self.partial_output,
+                self.output)
+        if ops.launches_directly(*args):
+            ops.launch_decode_attention(*args, self.splits, self.scale)
+            ops.mark_written(*args[4:])
+        else:
+            torch.ops.sfl.decode_attention(*args, self.splits, self.scale)
         return self.output
 
     @property

@@ -19,6 +19,28 @@ import torch
 from . import _lib
 
 
+def launches_directly(*tensors: torch.Tensor | None) -> bool:
+    """Whether an operator API may launch without going through the dispatcher.
+
+    Plain tensors outside every tracing, dispatch and differentiation mode
+    reach the kernels the same way either way; anything that wants to see or
+    transform the op (``torch.compile``, dispatch and function modes, functorch
+    transforms, forward-mode AD, the profiler, inputs that require grad) takes
+    the registered op. Its Python layers cost ~10 us of an operator call.
+    """
+    return not (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
+                or torch._C._len_torch_function_stack() or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch.autograd.forward_ad._current_level >= 0 or torch._C._autograd._profiler_enabled()
+                or any(t is not None and (type(t) is not torch.Tensor or t.requires_grad) for t in tensors))
+
+
+def mark_written(*tensors: torch.Tensor | None) -> None:
+    """Bump the version counters of tensors a direct launch wrote, as the op does."""
+    written = [t for t in tensors if t is not None and not t.is_inference()]
+    if written:
+        torch.autograd.graph.increment_version(written)
+
+
 def _strides(t: torch.Tensor):
     return (ctypes.c_long * 3)(t.stride(0), t.stride(1), t.stride(2))
 
@@ -27,9 +49,7 @@ def _ptr(t: torch.Tensor | None):
     return None if t is None else t.data_ptr()
 
 
-@torch.library.custom_op("sfl::decode_attention",
-                         mutates_args=("partial_max", "partial_sum", "partial_output", "out"))
-def decode_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, lengths: torch.Tensor,
+def launch_decode_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, lengths: torch.Tensor,
                      partial_max: torch.Tensor, partial_sum: torch.Tensor, partial_output: torch.Tensor,
                      out: torch.Tensor, splits: int, scale: float) -> None:
     """Split-KV decode attention into ``out`` [B, Hq, D] (``sfl_decode_attention``).
@@ -46,13 +66,17 @@ def decode_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, lengths:
               _lib.stream_handle(q.device))
 
 
+decode_attention = torch.library.custom_op(
+    "sfl::decode_attention", mutates_args=("partial_max", "partial_sum", "partial_output", "out"))(
+        launch_decode_attention)
+
+
 @decode_attention.register_fake
 def _decode_attention_fake(q, k, v, lengths, partial_max, partial_sum, partial_output, out, splits, scale):
     return None
 
 
-@torch.library.custom_op("sfl::masked_attention", mutates_args=("out", "lse"))
-def masked_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tensor,
+def launch_masked_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tensor,
                      lse: torch.Tensor | None, scale: float, causal: bool, window_left: int,
                      window_right: int, global_prefix: int, document_ids: torch.Tensor | None,
                      row_ptr: torch.Tensor | None, col_idx: torch.Tensor | None,
@@ -69,6 +93,10 @@ def masked_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: tor
               int(causal), window_left, window_right, global_prefix, _ptr(document_ids), mode,
               _ptr(row_ptr), _ptr(col_idx), _ptr(full_blocks), int(use_full_blocks),
               _lib.dtype_code(q.dtype), _lib.stream_handle(q.device))
+
+
+masked_attention = torch.library.custom_op("sfl::masked_attention", mutates_args=("out", "lse"))(
+    launch_masked_attention)
 
 
 @masked_attention.register_fake

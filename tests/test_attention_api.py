@@ -1,5 +1,7 @@
 """Host-side contract of the masked attention API (no GPU): rejections before any launch."""
 
+import dataclasses
+
 import pytest
 import torch
 
@@ -36,3 +38,14 @@ def test_schedule_validation():
         _validated_schedule(BlockSchedule(40, 16, 16, [0, 2, 2, 2], [1, 0], [False, False]))
     with pytest.raises(TypeError, match="bool"):
         _validated_schedule(BlockSchedule(5, 16, 16, [0, 1], [0], [1]))
+
+
+def test_schedule_entry_types_are_told_apart():
+    good = BlockSchedule(40, 16, 16, [0, 1, 2, 3], [0, 1, 2], [False, True, True])
+    _validated_schedule(good)
+    for field, value, error in (("row_ptr", True, TypeError), ("col_idx", 1.0, TypeError), ("col_idx", True, TypeError),
+                                ("full_blocks", 1, TypeError), ("col_idx", 1 << 31, ValueError)):
+        entries = list(getattr(good, field))
+        entries[1] = value
+        with pytest.raises(error):
+            _validated_schedule(dataclasses.replace(good, **{field: entries}))

@@ -91,3 +91,20 @@ def test_folded_norm_entry_points_reject_bad_arguments_without_a_launch():
         _lib.call("sfl_gemm_swiglu_scaled", p, p, p, p, 64, 100, 128, 1, None)
     with pytest.raises(RuntimeError, match="multiple of 64"):
         _lib.call("sfl_gemm_swiglu_scaled", p, p, p, p, 64, 128, 72, 1, None)
+
+
+def test_prefill_layers_rejects_before_any_launch():
+    import ctypes
+
+    from systems_for_llms_amd import _lib
+
+    one = (_lib.P * 1)(8)
+    sizes = dict(dtype=2, layers=1, batch=1, seq=4, d_model=64, heads=2, d_ff=64, capacity=4, fold=0, scale=1.0)
+    pointers = {name: one if kind is not _lib.P else 8 for name, kind in _lib.PrefillArgs._fields_
+                if name not in sizes}
+    assert _lib.lib().sfl_prefill_layers(None, None) != 0
+    for change in ({"x": None}, {"w_qkv": None}, {"layers": 0}, {"heads": 3}, {"seq": 1 << 30, "batch": 8},
+                   {"fold": 1, "ss": None}):
+        args = _lib.PrefillArgs(**{**sizes, **pointers, **change})
+        assert _lib.lib().sfl_prefill_layers(ctypes.addressof(args), None) != 0, change
+        assert "prefill_layers" in _lib.lib().sfl_last_error().decode()

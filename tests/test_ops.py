@@ -43,6 +43,54 @@ def test_meta_and_fake_dispatch_launch_nothing():
         torch.ops.sfl.decode_attention(*_decode_args("cpu"))
 
 
+def test_direct_launches_only_where_nothing_watches_the_op():
+    from systems_for_llms_amd.ops import launches_directly
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Watch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    seen, x = [], torch.zeros(2, 3)
+    assert launches_directly(x, None)
+    assert not launches_directly(x, x.clone().requires_grad_())
+    assert not launches_directly(torch.nn.Parameter(x, requires_grad=False))
+    with Watch():
+        seen.append(launches_directly(x))
+    with torch.overrides.BaseTorchFunctionMode():
+        seen.append(launches_directly(x))
+    with torch.autograd.forward_ad.dual_level():
+        seen.append(launches_directly(x))
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]):
+        seen.append(launches_directly(x))
+    torch.func.vmap(lambda row: (seen.append(launches_directly(x)), row)[1])(x)
+    torch.func.grad(lambda row: (seen.append(launches_directly(x)), row.sum())[1])(x)
+    assert seen == [False] * 6 and launches_directly(x)
+
+
+def test_mark_written_bumps_versions_like_the_op():
+    from systems_for_llms_amd.ops import mark_written
+
+    x, y = torch.zeros(2), torch.zeros(2)
+    mark_written(x, None, y)
+    assert x._version == 1 and y._version == 1
+    with torch.inference_mode():
+        mark_written(torch.zeros(2))  # inference tensors have no counter
+
+
+@pytest.mark.gpu
+def test_prepared_decode_bumps_the_output_version():
+    from systems_for_llms_amd.decode import prepare
+
+    q, k = torch.randn(1, 4, 64, device="cuda"), torch.randn(1, 4, 32, 64, device="cuda")
+    op = prepare(q, k, k.clone())
+    weight = torch.ones_like(q, requires_grad=True)
+    product = op() * weight  # saves the output for the backward
+    op()
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        product.sum().backward()
+
+
 @pytest.mark.gpu
 def test_decode_op_and_compiled_graph_match_oracle():
     from oracle.attention import decode_reference
