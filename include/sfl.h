@@ -399,21 +399,31 @@ int sfl_gemm_qkv_rope_normed(const void* a_xg, const void* w_qkv, const float* s
 int sfl_gemm_swiglu_normed(const void* a_xg, const void* w13_interleaved, const float* ss_parts, int parts,
                            void* h_out, int m, int d_ff, int k, int dtype, void* stream);
 
-/* ---- every layer of a prefill in one call ------------------------------------
+/* ---- a prefill in one call ----------------------------------------------------
  *
- * Launches, in order, sfl_embed_rows and each layer's sequence of the entry
- * points above: with fold (16-bit models only, d_model and d_ff multiples of
- * 64) the folded-norm ones, else sfl_rmsnorm_rows and the unscaled GEMMs; the
- * attention is causal (sfl_masked_attention on its interval schedule, fp32:
- * sfl_causal_attention_f32). x holds the last layer's output afterwards. The
- * pointer arrays are host arrays of one device pointer per layer; buffers as
- * the entry points describe them, in the model dtype unless typed. ss
+ * Loads the given tokens into the session's state and embeds the prompt (the
+ * first seq of them), launches each layer's sequence of the entry points above,
+ * and hands the last position over to the decode step:
+ *   tokens = given, then zeros; predicted = -1; prompt_len = given_len
+ *   layers: with fold (16-bit models only, d_model and d_ff multiples of 64)
+ *   the folded-norm entry points, else sfl_rmsnorm_rows and the unscaled GEMMs;
+ *   the attention is causal (sfl_masked_attention on its interval schedule,
+ *   fp32: sfl_causal_attention_f32)
+ *   x_last = the last layer's output at position seq - 1; pos = seq - 1;
+ *   lengths = seq
+ * x holds the last layer's output for every position afterwards. The pointer
+ * arrays are host arrays of one device pointer per layer; buffers as the entry
+ * points describe them, in the model dtype unless typed. ss
  * [max(ceil(d_model / part))][m] (fold; parts of sfl_gemm_norm_part) and
- * rscale [m] (fold) are scratch, m = batch * seq. */
+ * rscale [m] (fold) are scratch, m = batch * seq. d_model % 16 == 0, x and
+ * x_last 16-byte aligned. Token ids must be in the embedding's range. */
 typedef struct {
-  int dtype, layers, batch, seq, d_model, heads, d_ff, capacity, fold;
+  int dtype, layers, batch, seq, given_len, d_model, heads, d_ff, capacity, fold;
   float scale;                    /* attention: head_dim ^ -0.5 */
-  const int64_t* ids;             /* [m] */
+  const int64_t* given;           /* [batch, given_len], seq <= given_len <= capacity */
+  int64_t *tokens, *predicted;    /* [batch, capacity] */
+  int32_t *prompt_len, *pos, *lengths; /* [batch] */
+  float* x_last;                  /* [batch, d_model] */
   const void* emb;                /* [vocab, d_model] */
   const void* const* attn_norm;   /* [d_model] */
   const void* const* w_qkv;       /* [3 d_model, d_model] */

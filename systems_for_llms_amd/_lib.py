@@ -67,8 +67,10 @@ _LIB = None
 class PrefillArgs(ctypes.Structure):
     """``sfl_prefill_args`` of ``include/sfl.h``."""
 
-    _fields_ = ([(n, c_int) for n in ("dtype", "layers", "batch", "seq", "d_model", "heads", "d_ff", "capacity", "fold")]
-                + [("scale", c_float), ("ids", P), ("emb", P)]
+    _fields_ = ([(n, c_int) for n in ("dtype", "layers", "batch", "seq", "given_len", "d_model", "heads", "d_ff",
+                                      "capacity", "fold")]
+                + [("scale", c_float)]
+                + [(n, P) for n in ("given", "tokens", "predicted", "prompt_len", "pos", "lengths", "x_last", "emb")]
                 + [(n, POINTER(P)) for n in ("attn_norm", "w_qkv", "w_out", "ffn_norm", "w13", "w2", "k_cache",
                                              "v_cache")]
                 + [(n, P) for n in ("cos_t", "sin_t", "x", "act", "q", "attn", "hidden", "ss", "rscale")])

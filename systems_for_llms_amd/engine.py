@@ -340,24 +340,17 @@ class DecodeSession:
         weights = ([_weight(blk["attn_norm"]) for blk in blocks], self.wqkv,
                    [_weight(m["output_proj"]) for m in attns], [_weight(blk["ffn_norm"]) for blk in blocks], w13,
                    [_weight(m["w2"]) for m in ffns], self.k_cache.unbind(0), self.v_cache.unbind(0))
+        given = (prompt if forced is None else forced).to(dev, torch.int64).contiguous()
         args = _lib.PrefillArgs(
-            code, len(blocks), b, t, d, h, f, self.cap, int(fold), float(dk ** -0.5), None,
-            _weight(model.token_embeddings).data_ptr(), *map(_lib.pointers, weights), self.cos_fm.data_ptr(),
+            code, len(blocks), b, t, given.shape[1], d, h, f, self.cap, int(fold), float(dk ** -0.5), given.data_ptr(),
+            self.tokens.data_ptr(), self.predicted.data_ptr(), self.prompt_len.data_ptr(), self.pos.data_ptr(),
+            self.lengths.data_ptr(), self.x.data_ptr(), _weight(model.token_embeddings).data_ptr(), *map(_lib.pointers, weights), self.cos_fm.data_ptr(),
             self.sin_fm.data_ptr(), x.data_ptr(), act.data_ptr(), q.data_ptr(), attn.data_ptr(), hid.data_ptr(),
             _lib.ptr(ss), _lib.ptr(scale))
         low, high = bounds.tolist()
         if low < 0 or high >= self.vocab:
             raise ValueError("token ids must be in [0, vocab_size)")
         self.prefill_norm_folded = fold
-        self.tokens.zero_()
-        self.tokens[:, :t] = prompt.to(dev)
-        self.predicted.fill_(-1)
-        self.prompt_len.fill_(t)
-        if forced is not None:
-            self.tokens[:, :forced.shape[1]] = forced.to(dev)
-            self.prompt_len.fill_(forced.shape[1])
-        ids = self.tokens[:, :t].contiguous().view(-1)
-        args.ids = ids.data_ptr()
         _lib.call("sfl_prefill_layers", ctypes.addressof(args), st)
         logits = None
         if all_logits:
@@ -367,14 +360,11 @@ class DecodeSession:
             _lib.call("sfl_gemm", act.data_ptr(), _weight(model.lm_head).data_ptr(), logits.data_ptr(), m_rows, v, d,
                       code, _lib.dtype_code(logits_dtype), 0, st)
             logits = logits.view(b, t, v)
-        self._hand_over(x, b, t, st)
+        self._hand_over(t, st)
         return logits
 
-    def _hand_over(self, x, b, t, st) -> None:
-        """Hand the prompt's last position to the decode head: pick token T and advance."""
-        self.x.copy_(x.view(b, t, self.d)[:, t - 1])
-        self.pos.fill_(t - 1)
-        self.lengths.fill_(t)
+    def _hand_over(self, t, st) -> None:
+        """The decode head on the prompt's last position: pick token T and advance."""
         self.position = t
         for fn, args in self._calls[-2:]:  # the lm_head and the token step
             status = fn(*args, st)

@@ -98,13 +98,14 @@ def test_prefill_layers_rejects_before_any_launch():
 
     from systems_for_llms_amd import _lib
 
-    one = (_lib.P * 1)(8)
-    sizes = dict(dtype=2, layers=1, batch=1, seq=4, d_model=64, heads=2, d_ff=64, capacity=4, fold=0, scale=1.0)
-    pointers = {name: one if kind is not _lib.P else 8 for name, kind in _lib.PrefillArgs._fields_
+    one = (_lib.P * 1)(16)
+    sizes = dict(dtype=2, layers=1, batch=1, seq=4, given_len=4, d_model=64, heads=2, d_ff=64, capacity=4, fold=0, scale=1.0)
+    pointers = {name: one if kind is not _lib.P else 16 for name, kind in _lib.PrefillArgs._fields_
                 if name not in sizes}
     assert _lib.lib().sfl_prefill_layers(None, None) != 0
     for change in ({"x": None}, {"w_qkv": None}, {"layers": 0}, {"heads": 3}, {"seq": 1 << 30, "batch": 8},
-                   {"fold": 1, "ss": None}):
+                   {"fold": 1, "ss": None},
+                   {"given_len": 3}, {"given_len": 5}, {"d_model": 66}, {"x_last": 24}, {"dtype": 7}):
         args = _lib.PrefillArgs(**{**sizes, **pointers, **change})
         assert _lib.lib().sfl_prefill_layers(ctypes.addressof(args), None) != 0, change
         assert "prefill_layers" in _lib.lib().sfl_last_error().decode()

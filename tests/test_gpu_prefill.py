@@ -700,3 +700,35 @@ def test_f32_forward_is_one_prefill_pass_equal_to_the_oracle():
     b.run(239, use_graph=True)
     torch.cuda.synchronize()
     torch.testing.assert_close(a.logits[:, 200:239].cpu(), b.logits[:, 200:239].cpu(), atol=2e-5, rtol=1e-4)
+
+
+@pytest.mark.parametrize("batch,t,given,cap,offset", [(1, 1, 1, 1, 0), (3, 5, 5, 40, 0), (2, 7, 11, 11, 0), (5, 3, 4, 33, 0),
+                                                    (4, 6, 6, 6, 1)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_prefill_loads_the_session_state(batch, t, given, cap, offset, dtype):
+    """Tokens, predictions and counters after a prefill into a used session, and the embedded
+    prompt (through the logits), also from an embedding table off a 16-byte boundary."""
+    cfg = ModelConfig(vocab_size=97, context_length=64, d_model=64, num_layers=1, num_heads=2, d_ff=96)
+    model = gpu_model(cfg, seeded_state_dict(cfg, 3), dtype)
+    ids = torch.randint(0, 97, (batch, given), generator=torch.Generator().manual_seed(t))
+    plain = DecodeSession(model, batch, cap).prefill(ids[:, :t], all_logits=True)
+    if offset:
+        table = model.token_embeddings.weight
+        flat = torch.empty(table.numel() + offset, device="cuda", dtype=dtype)
+        flat[offset:].view_as(table).copy_(table.detach())
+        model.token_embeddings.weight.data = flat[offset:].view_as(table)
+    session = DecodeSession(model, batch, cap)
+    for name in ("tokens", "predicted", "pos", "lengths", "prompt_len"):
+        getattr(session, name).fill_(55)
+    logits = session.prefill(ids[:, :t].cuda(), all_logits=True, forced=ids if given > t else None)
+    torch.testing.assert_close(logits, plain, rtol=0, atol=0)
+    last = logits[:, -1].float().argmax(-1).cpu()
+    tokens, predicted = torch.zeros((batch, cap), dtype=torch.int64), torch.full((batch, cap), -1)
+    tokens[:, :given] = ids
+    if t < cap:  # the token step wrote position t
+        predicted[:, t] = session.predicted[:, t].cpu()
+        tokens[:, t] = ids[:, t] if given > t else predicted[:, t]
+        assert (predicted[:, t] == last).all()
+    assert torch.equal(session.tokens.cpu(), tokens) and torch.equal(session.predicted.cpu(), predicted)
+    at = t if t < cap else t - 1
+    assert (session.pos == at).all() and (session.lengths == at + 1).all() and (session.prompt_len == given).all()
