@@ -24,11 +24,12 @@ def launches_directly(*tensors: torch.Tensor | None) -> bool:
 
     Plain tensors outside every tracing, dispatch and differentiation mode
     reach the kernels the same way either way; anything that wants to see or
-    transform the op (``torch.compile``, dispatch and function modes, functorch
-    transforms, forward-mode AD, the profiler, inputs that require grad) takes
-    the registered op. Its Python layers cost ~10 us of an operator call.
+    transform the op (``torch.compile``, ``torch.jit.trace``, dispatch and
+    function modes, functorch transforms, forward-mode AD, the profiler, inputs
+    that require grad) takes the registered op. Its Python layers cost ~10 us of
+    an operator call.
     """
-    return not (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
+    return not (torch.compiler.is_compiling() or torch._C._is_tracing() or torch._C._len_torch_dispatch_stack()
                 or torch._C._len_torch_function_stack() or torch._C._functorch.peek_interpreter_stack() is not None
                 or torch.autograd.forward_ad._current_level >= 0 or torch._C._autograd._profiler_enabled()
                 or any(t is not None and (type(t) is not torch.Tensor or t.requires_grad) for t in tensors))

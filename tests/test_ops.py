@@ -65,7 +65,8 @@ def test_direct_launches_only_where_nothing_watches_the_op():
         seen.append(launches_directly(x))
     torch.func.vmap(lambda row: (seen.append(launches_directly(x)), row)[1])(x)
     torch.func.grad(lambda row: (seen.append(launches_directly(x)), row.sum())[1])(x)
-    assert seen == [False] * 6 and launches_directly(x)
+    torch.jit.trace(lambda row: (seen.append(launches_directly(row)), row + 1)[1], (x,), check_trace=False)
+    assert seen == [False] * 7 and launches_directly(x)
 
 
 def test_mark_written_bumps_versions_like_the_op():
