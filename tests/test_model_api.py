@@ -132,3 +132,16 @@ def test_checkpoint_errors(tmp_path):
     reference_style_checkpoint(path, wrong, state)
     with pytest.raises(RuntimeError, match="layers.2"):
         TransformerLM.from_checkpoint(path)
+
+
+def test_parameter_version_sees_changes_and_ends_on_cyclic_modules():
+    from systems_for_llms_amd.engine import parameter_version
+
+    cfg = ModelConfig(vocab_size=50, context_length=8, d_model=32, num_layers=2, num_heads=2, d_ff=64)
+    model = TransformerLM.from_config(cfg, device="cpu", dtype=torch.float32)
+    model.layers[0].owner = model
+    first = parameter_version(model)
+    assert first == parameter_version(model) and len(first) == len(list(model.parameters()))
+    with torch.no_grad():
+        model.layers[1].ffn.w2.weight.mul_(2)
+    assert parameter_version(model) != first
