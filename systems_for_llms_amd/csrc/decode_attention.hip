@@ -70,12 +70,12 @@ struct ProjShape {
   static constexpr int NCK = G * D >= KC ? G * D / KC : 1;
 };
 
-// Unit u of a wave's share: tile wave + (u / NCK) * W, chunk h * NCK + u % NCK.
-template <typename T, int D, int G, int W>
-__device__ __forceinline__ uint4 load_proj_unit(const unsigned char* w_lane, int u, int wave, int h,
+// Unit u of a wave's share: tile first + (u / NCK) * step, chunk h * NCK + u % NCK.
+template <typename T, int D, int G>
+__device__ __forceinline__ uint4 load_proj_unit(const unsigned char* w_lane, int u, int first, int step, int h,
                                                 int nchunks_all) {
   using P = ProjShape<T, D, G>;
-  const long tile = wave + (u / P::NCK) * W;
+  const long tile = first + (u / P::NCK) * step;
   const long c = long(h) * P::NCK + u % P::NCK;
   return load16(w_lane + (tile * nchunks_all + c) * kWave * 16);
 }
@@ -111,6 +111,9 @@ __global__ __launch_bounds__(W * kWave) void decode_attn_kernel(
   const int q_heads = kv_heads * G;
   const int slot = lane / LPT;
   const int dg = lane % LPT;
+  // Fused: always one split; `splits` is log2 of the workgroups (blockIdx.y)
+  // that share a head's output projection, each attending to the whole row.
+  const bool one_split = kProj || splits == 1;
 
   // The query does not depend on the length: issue its loads first.
   float qv[G][EPL];
@@ -134,7 +137,7 @@ __global__ __launch_bounds__(W * kWave) void decode_attn_kernel(
   // W/2 tiles of 8 loads (W tiles of 4), so a short row wastes at most that
   // much (with every wave speculating 8-load tiles: ~15.5 us per 324M launch
   // below length 1024 against ~11.5, and no faster at 3584).
-  const bool spec = splits == 1 && wave < W * 4 / NL;
+  const bool spec = one_split && wave < W * 4 / NL;
   uint4 kr[NL], vr[NL];
   if (spec) {
 #pragma unroll
@@ -143,7 +146,7 @@ __global__ __launch_bounds__(W * kWave) void decode_attn_kernel(
     for (int i = 0; i < NL; ++i) vr[i] = load16_stream(vb + long(min(t_first + i * TPL + slot, cap - 1)) * D);
   }
   const int len = min(max(lengths[b], 0), cap);
-  if (splits > 1 && begin >= len) return;  // the merge reads only chunks below the length
+  if (!one_split && begin >= len) return;  // the merge reads only chunks below the length
   const int end = min(len, begin + chunk);
   if (spec) {
 #pragma unroll
@@ -265,14 +268,16 @@ __global__ __launch_bounds__(W * kWave) void decode_attn_kernel(
   // Fused projection: issue the first round of W_o loads now, so they land
   // while the softmax states are merged. `out` is the packed W_o.
   const unsigned char* w_lane = static_cast<const unsigned char*>(out) + lane * 16;
-  const int proj_tiles = d_model / 16;
-  const int proj_units = kProj ? max(0, (proj_tiles - wave + W - 1) / W) * ProjShape<T, D, G>::NCK : 0;
+  const int proj_first = wave + (kProj ? int(blockIdx.y) * W : 0), proj_step = W << (kProj ? splits : 0);
+  const int proj_units =
+      kProj ? ((d_model / 16 - proj_first + proj_step - 1) / W >> splits) * ProjShape<T, D, G>::NCK : 0;
   uint4 wr[kProj ? kProjRound : 1];
   if constexpr (kProj) {
 #pragma unroll
     for (int j = 0; j < kProjRound; ++j)
       if (proj_units > 0)
-        wr[j] = load_proj_unit<T, D, G, W>(w_lane, min(j, proj_units - 1), wave, h, d_model / ProjShape<T, D, G>::KC);
+        wr[j] = load_proj_unit<T, D, G>(w_lane, min(j, proj_units - 1), proj_first, proj_step, h,
+                                        d_model / ProjShape<T, D, G>::KC);
   }
 
   // Merge the slots' online-softmax states: xor over the slot bits of the lane id.
@@ -337,7 +342,7 @@ __global__ __launch_bounds__(W * kWave) void decode_attn_kernel(
         const long qrow = long(b) * q_heads + h * G + g;
         if constexpr (kProj) {
           os[o] = den > 0.f ? num / den : 0.f;
-        } else if (splits == 1) {
+        } else if (one_split) {
           store_out<TO>(out, qrow * D + d, q_heads * D, den > 0.f ? num / den : 0.f);
         } else {
           const long prow = qrow * splits + split;
@@ -365,7 +370,7 @@ __global__ __launch_bounds__(W * kWave) void decode_attn_kernel(
       if (r0 > 0) {
 #pragma unroll
         for (int j = 0; j < kProjRound; ++j)
-          wr[j] = load_proj_unit<T, D, G, W>(w_lane, min(r0 + j, proj_units - 1), wave, h, d_model / P::KC);
+          wr[j] = load_proj_unit<T, D, G>(w_lane, min(r0 + j, proj_units - 1), proj_first, proj_step, h, d_model / P::KC);
       }
 #pragma unroll
       for (int j = 0; j < kProjRound; ++j) {
@@ -379,7 +384,7 @@ __global__ __launch_bounds__(W * kWave) void decode_attn_kernel(
           if (u % P::NCK == P::NCK - 1) {
             part += lane_xor(part, 16);
             part += lane_xor(part, 32);
-            const int tile = wave + (u / P::NCK) * W;
+            const int tile = proj_first + (u / P::NCK) * proj_step;
             if (lane < 16) unsafeAtomicAdd(xb + tile * 16 + lane, part);
             part = 0.f;
           }
@@ -739,6 +744,25 @@ inline bool gqa_mfma_fits(const DecodeCall& c) {
   return a16(c.q) && a16(c.k) && a16(c.v) && long(c.cap) * c.dim * 2 < (1L << 31);
 }
 
+// log2 of the workgroups that share one head's output projection. A short batch
+// has a workgroup (of the whole chip's 256 CUs) per head, which pulls the head's
+// d_model columns of W_o through one CU beside its keys: with 2 or 4 workgroups
+// that each attend to the whole row (its second reader finds the row in L2 or
+// the MALL) and project a part of the outputs, the launch is shorter as long as
+// each still has a CU of its own, longer beyond. us at 1 / 2 / 4 / 8 workgroups
+// (bf16, D 64, weights and caches from HBM):
+//   batch 1, 16 heads, 611 keys   8.7 /  8.0 /  7.6 /  7.6
+//   batch 1, 16 heads, 3583 keys 22.9 / 21.3 / 20.3 / 19.6
+//   batch 1, 12 heads, 611 keys   8.2 /  8.2 /  7.8 /  7.8 (fp16)
+//   batch 4, 16 heads, 500 keys   8.7 /  8.0 /  7.8 / 12.4 (8: 512 workgroups)
+//   batch 8, 16 heads, 3583 keys 27.1 / 27.0 / 52.7 (4: 512 workgroups)
+// A wave keeps at least half a tile of the projection.
+inline int proj_share_log2(long groups, int waves, int tiles) {
+  int share = 0;
+  while (share < 2 && (groups << (share + 1)) <= 256 && (waves << (share + 1)) <= 2 * tiles) ++share;
+  return share;
+}
+
 template <typename T, typename TQ, typename TO, int D, int G>
 int launch_attn(const DecodeCall& c) {
   if constexpr (gqa_mfma_shape<T, TQ, TO, D, G>()) {
@@ -755,9 +779,14 @@ int launch_attn(const DecodeCall& c) {
   constexpr int W = waves_for<T, D, G>();
   const int chunk = (c.cap + c.splits - 1) / c.splits;
   const long groups = long(c.batch) * c.kv_heads * c.splits;
-  hipLaunchKernelGGL((decode_attn_kernel<T, TQ, TO, D, G, W>), dim3(unsigned(groups)), dim3(W * kWave), 0,
-                     c.stream, static_cast<const TQ*>(c.q), static_cast<const T*>(c.k),
-                     static_cast<const T*>(c.v), c.lengths, c.kv_heads, c.cap, c.splits, chunk,
+  int splits = c.splits, share = 0;
+  if constexpr (std::is_same<TO, resid_t>::value) {
+    share = proj_share_log2(groups, W, c.d_model / 16);
+    splits = share;
+  }
+  hipLaunchKernelGGL((decode_attn_kernel<T, TQ, TO, D, G, W>), dim3(unsigned(groups), 1u << share),
+                     dim3(W * kWave), 0, c.stream, static_cast<const TQ*>(c.q), static_cast<const T*>(c.k),
+                     static_cast<const T*>(c.v), c.lengths, c.kv_heads, c.cap, splits, chunk,
                      c.scale * kLog2e, c.d_model, c.pmax, c.psum, c.pout, c.out, c.x);
   return check_launch("decode_attention");
 }

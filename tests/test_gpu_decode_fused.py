@@ -112,6 +112,15 @@ def test_attention_out_proj_matches_reference(dtype, dim, batch, heads):
         torch.testing.assert_close(got[1], x0[1].double(), atol=0, rtol=0)
 
 
+# Workgroups per head's projection: 4 with more of them than tiles (48 tiles, 64 waves), 4 at the limit of
+# 256 workgroups, 2, and 2 of 8 waves.
+@pytest.mark.parametrize("dtype,dim,batch,heads", [(torch.float16, 64, 1, 12), (torch.bfloat16, 64, 4, 16),
+                                                   (torch.bfloat16, 32, 5, 20), (torch.float32, 64, 8, 16),
+                                                   (torch.bfloat16, 128, 11, 9)])
+def test_attention_out_proj_shared_by_workgroups(dtype, dim, batch, heads):
+    test_attention_out_proj_matches_reference(dtype, dim, batch, heads)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_attention_out_proj_long_ragged_rows(dtype):
     """Rows several key tiles per wave long (head dim 64: the tile loop with one tile of loads ahead),
