@@ -295,11 +295,18 @@ int sfl_masked_attention_kernel_info(int head_dim, int dtype, int n, long k_row_
  * C^T = W A^T on MFMAs; A [M, K] row-major (one row per token) and W [N, K]
  * of one type `dtype`: SFL_DTYPE_BF16 or SFL_DTYPE_F16 (16-bit MFMAs; every
  * 16-bit output of these calls has that type too; K % 8 == 0; K % 64 == 0 runs
- * 32x32x16 MFMA tiles of 256 x 384 (grids of >= 320 such tiles) or 128 x 128
- * features x tokens, other K the 16x16x32 kernel on 128 x 128 tiles), or, for
- * sfl_gemm, sfl_gemm_qkv_rope and sfl_gemm_swiglu, SFL_DTYPE_F32 (fp32
- * v_mfma_f32_32x32x2_f32 on 64 x 64 tiles: fp32 products and sums, every
- * output fp32, K % 4 == 0, 16-byte aligned operands and outputs).
+ * 32x32x16 MFMAs on tiles of 32 x 32 up to 256 x 384 features x tokens,
+ * whichever suits the grid, other K the 16x16x32 kernel on 128 x 128 tiles),
+ * or, for sfl_gemm, sfl_gemm_qkv_rope and sfl_gemm_swiglu, SFL_DTYPE_F32
+ * (every output fp32, K % 4 == 0, 16-byte aligned operands and outputs; sums
+ * in fp32). fp32 products: with K % 32 == 0 and operands under
+ * 2^29 elements each operand is split into three bf16 pieces, exactly, and eight
+ * of the nine products of two operands' pieces are summed on the bf16 matrix
+ * cores; the ninth is below 2^-30 of the product, a rounding of it 2^-24. Output
+ * tiles with an infinity, a NaN or an operand under 2^-110 that the pieces do
+ * not hold, and other K and sizes, run on v_mfma_f32_32x32x2_f32.
+ * The order in which a row's products are added depends on the tile, so on m:
+ * equal rows in batches of other sizes agree to rounding, not bit for bit.
  * Replace, for a whole prompt, the Linear layers of one TransformerBlock and
  * the lm_head (src/llmlab/model/layers.py:34-35, attention.py:160-162,199-203,
  * layers.py:114-115, transformer.py:137-138).
@@ -329,8 +336,9 @@ int sfl_gemm_swiglu(const void* a, const void* w13_interleaved, void* h_out, int
  * causal mask of :187-197), for the prefill of float32 models: q, k, v, o
  * [B, H, N, D] fp32 addressed by per-tensor strides {batch, head, sequence}
  * (elements; D contiguous; k, v and o rows 16-byte aligned), o = softmax(q k^T
- * * scale) v over keys 0..i for query i, every product and sum in fp32.
- * D in {16, 32, 64, 128}. */
+ * * scale) v over keys 0..i for query i, the products as for sfl_gemm with
+ * SFL_DTYPE_F32 (on the VALU where the pieces do not serve), every sum and the
+ * softmax in fp32. D in {16, 32, 64, 128}. */
 int sfl_causal_attention_f32(const float* q, const float* k, const float* v, float* o, int batch, int heads,
                              int n, int head_dim, const long* q_strides, const long* k_strides,
                              const long* v_strides, const long* o_strides, float scale, void* stream);

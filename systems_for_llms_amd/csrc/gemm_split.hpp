@@ -27,17 +27,25 @@ __device__ __forceinline__ f32x16 mma_slot(const u32x4& a, const u32x4& b, f32x1
 }
 
 
-// fp32 products on the bf16 matrix cores: 8 floats as three bf16 pieces each,
-// x = p0 + p1 + p2 exactly (8 significant bits apiece by truncation, all of
-// x's sign), of whose nine products the six with p0 p0 .. p1 p1, p0 p2 are
-// summed in fp32 (the other three are below 2^-21 of the product, 2^-24 on
-// average). An MFMA
-// takes 16 k values at 32 cycles, six of them 192, where eight 32x32x2 fp32
-// ones take 512; and with fewer, larger steps the sums round less: against
-// float64 the relative error (2-norm) is 1.8e-7 at K = 512, 2.2e-7 at 768,
-// 4.1e-7 at 2752, with fp32 MFMAs here 2.1e-7, 2.5e-7, 4.7e-7, in one chain
-// over K (gemm_f32_kernel) 4.1e-7, 5.0e-7, 9.4e-7.
-__device__ __forceinline__ void split3(const uint4& lo, const uint4& hi, u32x4 (&p)[3]) {
+// fp32 products on the bf16 matrix cores, by the published method of splitting
+// an fp32 operand into three bf16 ones (Henry, Tang, Heinecke, "Leveraging the
+// bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations",
+// ARITH 2019): x = p0 + p1 + p2 exactly, 8 significant bits apiece by
+// truncation, all of x's sign. Of the nine products of two operands' pieces the
+// eight without p2 p2 are summed in fp32; the one left out is below 2^-30 of
+// the operands' product, under the 2^-24 that an fp32 product rounds by. p0 p0
+// has a sum of its own: the other seven, at most 2^-6 of it, then cost it one
+// rounding in all and not one per product, so a sum of few terms is as exact as
+// one of fp32 products.
+// `lost` collects the bits no piece holds in its low half: none for operands
+// of at least 2^-110, some below, where p2 would need values under bf16's
+// smallest subnormal (the MFMAs keep subnormal operands and results); the
+// callers compute such a tile again on fp32 products. (No contraction: the
+// remainder is that of x, not of a product x was rounded from.)
+// An MFMA takes 16 k values at 32 cycles, eight of them 256, where eight
+// 32x32x2 fp32 ones take 512.
+__device__ __forceinline__ void split3(const uint4& lo, const uint4& hi, u32x4 (&p)[3], uint32_t& lost) {
+#pragma clang fp contract(off)
   const uint32_t x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -50,14 +58,22 @@ __device__ __forceinline__ void split3(const uint4& lo, const uint4& hi, u32x4 (
         b = __float_as_uint(__uint_as_float(b) - __uint_as_float(b & 0xffff0000u));
       }
     }
+    lost |= a | b;
   }
 }
+
+// The products beside p0 p0, smallest first: piece kLowA[i] of one operand with
+// piece kLowB[i] of the other.
+constexpr int kLowProducts = 7;
+constexpr int kLowA[kLowProducts] = {2, 1, 2, 1, 0, 1, 0};
+constexpr int kLowB[kLowProducts] = {1, 2, 0, 1, 2, 0, 1};
 
 // TBN features x TBM tokens per workgroup of NW waves; wave w takes the KS-wide
 // K chunks w, w + NW, ... of the whole tile through a private ring of NS LDS
 // stages (the layout, swizzle and operand reads of gemm32_kernel's stages).
 template <typename T, int E, int TBN, int TBM, int KS, int NW, int NS>
-__global__ __launch_bounds__(NW * kWave) void gemm_split_kernel(typename SplitArgs<T>::type g) {
+__global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(std::is_same<T, float>::value ? 2 : 1)))
+void gemm_split_kernel(typename SplitArgs<T>::type g) {
   constexpr bool kF32 = std::is_same<T, float>::value;
   constexpr int EB = Elem<T>::bytes;            // bytes per operand element
   constexpr int NBN = TBN / 32, NBM = TBM / 32, NB = NBN * NBM;  // 32x32 blocks of the tile
@@ -95,8 +111,18 @@ __global__ __launch_bounds__(NW * kWave) void gemm_split_kernel(typename SplitAr
   };
 
   f32x16 acc[NBN][NBM];
+  f32x16 low[kF32 ? NBN : 1][kF32 ? NBM : 1];  // fp32: the products beside p0 p0
   const int mine = (chunks - wave + NW - 1) / NW;  // this wave's chunks
   const int sw = stage_swizzle<SL>(l32);
+  uint32_t lost = 0;
+  if constexpr (kF32) {
+#pragma unroll
+    for (int i = 0; i < NBN; ++i)
+#pragma unroll
+      for (int j = 0; j < NBM; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) low[i][j][e] = 0.f;
+  }
   const auto k_loop = [&](auto pieces) {
 #pragma unroll
     for (int i = 0; i < NBN; ++i)
@@ -118,16 +144,19 @@ __global__ __launch_bounds__(NW * kWave) void gemm_split_kernel(typename SplitAr
           const int slot = 4 * kk + 2 * hf;
           u32x4 af[NBN][3], bf[NBM][3];
 #pragma unroll
-          for (int i = 0; i < NBN; ++i) split3(s.w[32 * i + l32][slot ^ sw], s.w[32 * i + l32][(slot + 1) ^ sw], af[i]);
+          for (int i = 0; i < NBN; ++i) split3(s.w[32 * i + l32][slot ^ sw], s.w[32 * i + l32][(slot + 1) ^ sw], af[i], lost);
 #pragma unroll
-          for (int j = 0; j < NBM; ++j) split3(s.a[32 * j + l32][slot ^ sw], s.a[32 * j + l32][(slot + 1) ^ sw], bf[j]);
-          constexpr int pa[6] = {2, 1, 0, 1, 0, 0}, pb[6] = {0, 1, 2, 0, 1, 0};  // smallest products first
+          for (int j = 0; j < NBM; ++j) split3(s.a[32 * j + l32][slot ^ sw], s.a[32 * j + l32][(slot + 1) ^ sw], bf[j], lost);
 #pragma unroll
-          for (int p = 0; p < 6; ++p)
+          for (int p = 0; p < kLowProducts; ++p)
 #pragma unroll
             for (int i = 0; i < NBN; ++i)
 #pragma unroll
-              for (int j = 0; j < NBM; ++j) acc[i][j] = mfma32<bf16_t>(af[i][pa[p]], bf[j][pb[p]], acc[i][j]);
+              for (int j = 0; j < NBM; ++j) low[i][j] = mfma32<bf16_t>(af[i][kLowA[p]], bf[j][kLowB[p]], low[i][j]);
+#pragma unroll
+          for (int i = 0; i < NBN; ++i)
+#pragma unroll
+            for (int j = 0; j < NBM; ++j) acc[i][j] = mfma32<bf16_t>(af[i][0], bf[j][0], acc[i][j]);
         }
       } else {
 #pragma unroll
@@ -158,15 +187,19 @@ __global__ __launch_bounds__(NW * kWave) void gemm_split_kernel(typename SplitAr
     k_loop(std::true_type{});
     // An infinite or NaN operand leaves a NaN remainder, so every sum it
     // enters is NaN: such a tile is computed again on fp32 products, whose
-    // infinities and NaNs are those of the operation.
-    bool nan = false;
+    // infinities and NaNs are those of the operation, and so is one with an
+    // operand its pieces do not hold.
+    bool redo = (lost & 0xffffu) != 0;
 #pragma unroll
     for (int i = 0; i < NBN; ++i)
 #pragma unroll
       for (int j = 0; j < NBM; ++j)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) nan |= acc[i][j][e] != acc[i][j][e];
-    if (__syncthreads_or(nan)) k_loop(std::false_type{});
+        for (int e = 0; e < 16; ++e) {
+          acc[i][j][e] += low[i][j][e];
+          redo |= acc[i][j][e] != acc[i][j][e];
+        }
+    if (__syncthreads_or(redo)) k_loop(std::false_type{});
   } else {
     k_loop(std::false_type{});
   }

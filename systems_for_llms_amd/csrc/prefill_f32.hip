@@ -4,12 +4,14 @@
 // The reference's float32 TransformerLM.forward (src/llmlab/model/
 // transformer.py:121-139) runs every Linear (layers.py:34-35) and the
 // attention (attention.py:61-98,187-197) in fp32; these kernels form every
-// product of fp32 values to at least fp32 accuracy and sum in fp32, so they
+// product of fp32 values to within an fp32 rounding and sum in fp32, so they
 // differ from it by the order of fp32 additions.
 //
 // GEMM: K a multiple of 32 and operands under 2 GiB run gemm_split_kernel
-// (gemm_split.hpp: K split over the waves, each fp32 product formed exactly
-// from bf16 pieces on the bf16 matrix cores). Other shapes run
+// (gemm_split.hpp: K split over the waves, each operand as three exact bf16
+// pieces, eight of whose nine products are summed on the bf16 matrix cores;
+// the ninth is below 2^-30 of the product). Its tiles with an infinity, a NaN
+// or an operand under 2^-110 are computed again on fp32 MFMAs. Other shapes run
 // gemm_f32_kernel: C^T[n][m] = sum_k W[n][k] A[m][k] on v_mfma_f32_32x32x2_f32
 // (fp32 operands, fp32 accumulation). A workgroup of 4 waves (2 x 2) computes 64
 // features x 64 tokens, a wave one 32 x 32 block; K advances by 32 through two
@@ -181,22 +183,24 @@ __device__ __forceinline__ void causal_rows_valu(const F32AttnArgs& a, int qb, i
 }
 
 // Causal attention of 64 queries per workgroup on the bf16 matrix cores, every
-// fp32 operand as three exact bf16 pieces (split3), six products each: S^T =
+// fp32 operand as three exact bf16 pieces, eight products each (split3): S^T =
 // K Q^T and O^T += V^T P^T with the layouts of the 16-bit masked attention
 // (k_swizzle, vt_slot, transpose reads), K and V split once per tile into
 // three LDS planes. Waves 0 and 1 take the first 32 keys of each 64-key tile
 // for queries 0..31 and 32..63, waves 2 and 3 the other 32 keys: a wave's
 // chain -- the longest row bounds a short launch -- is half as long, and the
 // two halves of a row merge through LDS at the end. The softmax is fp32, the
-// row sum over the fp32 probabilities. Against the VALU kernel this replaces
-// (one key at a time, 21 TFLOP/s), causal us: 4x12x1000 D 64 276 -> 58,
-// 2x16x4096 D 64 2215 -> 440, 8x16x256 D 32 53 -> 13, 2x4x2048 D 128
-// 760 -> 145; relative error to float64 3.3e-7 -> 2.5e-7, 5.7e-7 -> 3.4e-7,
-// 2.0e-7 -> 1.6e-7, 4.4e-7 -> 3.3e-7. Bound by the split and softmax VALU work
-// beside ~1500 MFMA cycles per 32 x 32 block at D 64; 3 waves per SIMD there
-// spill (50 registers). A row that comes out NaN (an infinity or NaN
-// in q, k or v, which the pieces do not carry, or which a masked key's zero
-// probability would multiply) sends its workgroup to causal_rows_valu.
+// row sum over the fp32 probabilities (v_exp_f32 gives 0 for one below 2^-126
+// of the row's largest, and its pieces keep what is at least 2^-133). Against
+// causal_rows_valu for every row (one key at a time, 21 TFLOP/s), causal us:
+// 4x12x1000 D 64 272 -> 62, 2x16x4096 D 64 2220 -> 509, 8x16x256 D 32
+// 50 -> 12.5, 2x4x2048 D 128 758 -> 166; relative error to float64 (2-norm)
+// 3.3e-7 -> 1.3e-7 at 4x12x1000, 2.0e-7 -> 1.0e-7 at 8x16x256. Bound by the
+// split and softmax VALU work beside ~2000 MFMA cycles per 32 x 32 block at
+// D 64; 3 waves per SIMD there do not fit its 230 registers. A row that comes
+// out NaN (an infinity or NaN in q, k or v, which the pieces do not carry, or
+// which a masked key's zero probability would multiply) or an operand its
+// pieces do not hold sends its workgroup to causal_rows_valu.
 template <int D>
 __global__ __launch_bounds__(kF32Threads) __attribute__((amdgpu_waves_per_eu(D < 64 ? 3 : D == 64 ? 2 : 1)))
 void causal_attention_f32_kernel(F32AttnArgs a) {
@@ -224,6 +228,7 @@ void causal_attention_f32_kernel(F32AttnArgs a) {
 
   // Q^T operand pieces of step ks: dims (D/2) h + 8 ks .. +7, scaled.
   u32x4 qreg[KS][3];
+  uint32_t lost = 0;
   {
     const float* qp = a.q + b * a.qs[0] + hd * a.qs[1] + long(min(qrow, a.n - 1)) * a.qs[2] + (D / 2) * h;
 #pragma unroll
@@ -231,7 +236,7 @@ void causal_attention_f32_kernel(F32AttnArgs a) {
       uint32_t x[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) x[e] = __float_as_uint(qp[8 * ks + e] * a.scale_log2);
-      split3(make_uint4(x[0], x[1], x[2], x[3]), make_uint4(x[4], x[5], x[6], x[7]), qreg[ks]);
+      split3(make_uint4(x[0], x[1], x[2], x[3]), make_uint4(x[4], x[5], x[6], x[7]), qreg[ks], lost);
     }
   }
   const float* kb = a.k + b * a.ks[0] + hd * a.ks[1];
@@ -255,7 +260,12 @@ void causal_attention_f32_kernel(F32AttnArgs a) {
   for (int t = 0; t < DT; ++t) vlane[t] = vt_lane_offset<DL>(lane, t) + unsigned(grp) * 32u * 2u * DL;
 
   float m_run = -INFINITY, l_run = 0.f;
-  f32x16 o[DT];
+  // The products beside p0 p0 of one dim tile: a running sum of their own, or,
+  // of several dim tiles, one per step (registers).
+  constexpr bool kLowKept = DT == 1;
+  f32x16 o[DT], o_low, zero;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) o_low[j] = zero[j] = 0.f;
 #pragma unroll
   for (int t = 0; t < DT; ++t)
 #pragma unroll
@@ -269,8 +279,8 @@ void causal_attention_f32_kernel(F32AttnArgs a) {
       if (kAttnK * SL % kF32Threads == 0 || idx < kAttnK * SL) {
         const int r = idx / SL, s = idx % SL;
         u32x4 pk[3], pv[3];
-        split3(kr[i][0], kr[i][1], pk);
-        split3(vr[i][0], vr[i][1], pv);
+        split3(kr[i][0], kr[i][1], pk, lost);
+        split3(vr[i][0], vr[i][1], pv, lost);
 #pragma unroll
         for (int p = 0; p < 3; ++p) {
           st.k[p][r][s ^ k_swizzle<DL>(r)] = make_uint4(pk[p][0], pk[p][1], pk[p][2], pk[p][3]);
@@ -281,10 +291,9 @@ void causal_attention_f32_kernel(F32AttnArgs a) {
     __syncthreads();
     if (t < qb) load(t + 1);
     if (t == qb && grp > qsub) continue;  // keys above every query of the wave
-    constexpr int pa[6] = {2, 1, 0, 1, 0, 0}, pb[6] = {0, 1, 2, 0, 1, 0};  // smallest products first
-    f32x16 s;
+    f32x16 s, s_low;
 #pragma unroll
-    for (int j = 0; j < 16; ++j) s[j] = 0.f;
+    for (int j = 0; j < 16; ++j) s[j] = s_low[j] = 0.f;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       u32x4 kp[3];
@@ -294,8 +303,10 @@ void causal_attention_f32_kernel(F32AttnArgs a) {
         kp[p] = u32x4{r.x, r.y, r.z, r.w};
       }
 #pragma unroll
-      for (int p = 0; p < 6; ++p) s = mfma32<bf16_t>(kp[pa[p]], qreg[ks][pb[p]], s);
+      for (int p = 0; p < kLowProducts; ++p) s_low = mfma32<bf16_t>(kp[kLowA[p]], qreg[ks][kLowB[p]], s_low);
+      s = mfma32<bf16_t>(kp[0], qreg[ks][0], s);
     }
+    s += s_low;
     if (t == qb && grp == qsub) {  // the diagonal block (attention.py:187-197)
 #pragma unroll
       for (int j = 0; j < 16; ++j) s[j] = 8 * (j / 4) + 4 * h + j % 4 <= c ? s[j] : -INFINITY;
@@ -317,6 +328,7 @@ void causal_attention_f32_kernel(F32AttnArgs a) {
     if (__ballot(alpha != 1.f)) {
 #pragma unroll
       for (int d = 0; d < DT; ++d) o[d] *= alpha;
+      if (kLowKept) o_low *= alpha;
     }
 #pragma unroll
     for (int s2 = 0; s2 < 2; ++s2) {
@@ -324,7 +336,8 @@ void causal_attention_f32_kernel(F32AttnArgs a) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) x[e] = __float_as_uint(s[8 * s2 + e]);
       u32x4 pp[3];
-      split3(make_uint4(x[0], x[1], x[2], x[3]), make_uint4(x[4], x[5], x[6], x[7]), pp);
+      uint32_t below = 0;  // of a probability, only what is under 2^-133 of the row's largest
+      split3(make_uint4(x[0], x[1], x[2], x[3]), make_uint4(x[4], x[5], x[6], x[7]), pp, below);
 #pragma unroll
       for (int d = 0; d < DT; ++d) {
         u32x4 vp[3];
@@ -337,13 +350,17 @@ void causal_attention_f32_kernel(F32AttnArgs a) {
           vp[p] = u32x4{l2.x, l2.y, h2.x, h2.y};
         }
 #pragma unroll
-        for (int p = 0; p < 6; ++p) o[d] = mfma32<bf16_t>(vp[pa[p]], pp[pb[p]], o[d]);
+        for (int p = 0; p < kLowProducts; ++p)
+          o_low = mfma32<bf16_t>(vp[kLowA[p]], pp[kLowB[p]], kLowKept || p ? o_low : zero);
+        o[d] = mfma32<bf16_t>(vp[0], pp[0], o[d]);
+        if (!kLowKept) o[d] += o_low;
       }
     }
   }
 
   // Waves 2 and 3 hand their half of each row to waves 0 and 1.
   l_run += lane_xor(l_run, 32);
+  if (kLowKept) o[0] += o_low;
   float* const red = reinterpret_cast<float*>(&st) + (qsub * (16 * DT + 2)) * kWave + lane;
   __syncthreads();
   if (grp == 1) {
@@ -355,7 +372,7 @@ void causal_attention_f32_kernel(F32AttnArgs a) {
     red[(16 * DT + 1) * kWave] = l_run;
   }
   __syncthreads();
-  bool nan = false;
+  bool redo = (lost & 0xffffu) != 0;
   if (grp == 0) {
     const float m1 = red[16 * DT * kWave], l1 = red[(16 * DT + 1) * kWave];
     const float top = fmaxf(m_run, m1);
@@ -366,10 +383,10 @@ void causal_attention_f32_kernel(F32AttnArgs a) {
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         o[d][j] = (o[d][j] * w0 + red[(16 * d + j) * kWave] * w1) * inv;
-        if (D >= 32 || j < 8) nan |= o[d][j] != o[d][j];
+        if (D >= 32 || j < 8) redo |= qrow < a.n && o[d][j] != o[d][j];
       }
   }
-  if (__syncthreads_or(nan && qrow < a.n)) return causal_rows_valu<D>(a, qb, b, hd, reinterpret_cast<float*>(&st));
+  if (__syncthreads_or(redo)) return causal_rows_valu<D>(a, qb, b, hd, reinterpret_cast<float*>(&st));
   if (grp == 1 || qrow >= a.n) return;
   float* op = a.o + b * a.os[0] + hd * a.os[1] + long(qrow) * a.os[2];
 #pragma unroll
@@ -393,11 +410,12 @@ int launch_tile(const F32GemmArgs& g, hipStream_t s, const char* what) {
 // covers the grid no larger tile is faster; 64 x 64 on 8 waves fills a CU
 // alone; beyond, 64 x 64 (two per CU) or 64 x 32 (three), whichever leaves the
 // fullest CU less to do (a 64 x 32 tile costs 1.12 halves of a 64 x 64 one).
-// us, gemm_f32_kernel -> this: M 1000 N 512 K 512 19.6 -> 8.8 (32 x 32);
-// M 2048 N 512 K 1344 63 -> 22 (64 x 64, 8 waves); M 1000 N 2304 K 768
-// 57 -> 33 (64 x 32; 64 x 64 34); M 4000 N 2304 K 768 162 -> 95, M 12000 N 4096
-// K 768 749 -> 483 (64 x 64: 156 TFLOP/s). 128 x 64 and 128 x 128 gain only at
-// K = 2752 (7-11%).
+// us, gemm_f32_kernel -> this: M 1000 N 512 K 512 18.0 -> 8.7 (32 x 32);
+// M 2048 N 512 K 1344 61 -> 25 (64 x 64, 8 waves); M 1000 N 2304 K 768
+// 56 -> 37 (64 x 32); M 4000 N 2304 K 768 155 -> 111, M 12000 N 4096 K 768
+// 730 -> 559 (64 x 64: 135 TFLOP/s). Relative error to float64 (2-norm) at
+// K 64 / 512 / 768 / 2752: 1.5 / 4.1 / 5.0 / 9.4e-7 -> 0.5 / 0.8 / 0.9 / 1.5e-7;
+// of a row with one non-zero value, 2.5e-8 rms and 6.0e-8 at most either way.
 template <int E>
 int launch_split(const F32GemmArgs& g, hipStream_t s, const char* what) {
   constexpr long kCus = 256;

@@ -1,6 +1,6 @@
 """float32 causal attention at the edges of its tiles and with infinities and NaN.
 
-Tolerance: scores are fp32 sums of D products kept to 2^-21, scaled to log2
+Tolerance: scores are fp32 sums of D products kept to 2^-24, scaled to log2
 units: their error is below e_s = (D + 9) 2^-24 sum |q k| log2(e) D^-1/2, and a
 probability's relative error below e_s + 2^-22; numerator and denominator each
 add n roundings of 2^-24, so an output is within
@@ -64,3 +64,17 @@ def test_infinities_and_nan_stay_with_their_rows(d):
     assert torch.equal(got[want.isinf()], want[want.isinf()])
     finite = want.isfinite()
     torch.testing.assert_close(got[finite], want[finite], atol=2e-5, rtol=2e-5)
+
+
+@pytest.mark.parametrize("d", [16, 64, 128])
+def test_values_and_queries_near_the_smallest(d):
+    """Operands whose 24 bits reach below the smallest bf16 subnormal keep all of them, and one
+    admissible key gives its value back bit for bit."""
+    q, k, v = inputs(2, 3, 100, d, 5)
+    q[0], k[0] = q[0] * 2.0 ** -115, k[0] * 2.0 ** 115
+    v[:, 1] *= 2.0 ** -118
+    e_s = ((q.abs() @ k.abs().transpose(-1, -2)).max() * (d + 9) * 2.0 ** -24 * 1.4427 * d ** -0.5).item()
+    got, want = run(q, k, v), rows_in_float64(q, k, v)
+    bound = (2 * e_s + (2 * 100 + 32) * 2.0 ** -24) * v.abs().amax((2, 3), keepdim=True).double()
+    assert ((got - want).abs() <= bound).all()
+    assert torch.equal(got[:, :, 0], v[:, :, 0].double())

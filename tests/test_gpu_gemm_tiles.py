@@ -125,8 +125,8 @@ def test_normed_consumers(batch, seq, d, heads, d_ff, dtype):
 @pytest.mark.parametrize("m,n,k", [(1, 40, 32), (33, 1000, 96), (65, 512, 1344), (500, 1536, 512), (1000, 520, 64),
                                    (513, 2304, 768), (2049, 1030, 96), (300, 264, 36), (4000, 2312, 32)])
 def test_fp32(m, n, k):
-    """float32 GEMM: sums of products kept to 2^-21 (three products of 16-bit remainders left
-    out, each at most 2^-22) at the edges of its tiles, accumulation and SwiGLU included."""
+    """float32 GEMM at the edges of its tiles, accumulation and SwiGLU included: (K + 9) 2^-24
+    sum |a w|, each product off by less than 2^-24 and each addition by half a unit."""
     from systems_for_llms_amd import _lib
 
     a, w = operands(m, n, k, torch.float32)
@@ -167,6 +167,43 @@ def test_fp32_special_values(m, n, k):
     assert ((out.double() - want).abs()[finite] <= bound[finite]).all()
     assert torch.equal(out.isnan(), want.isnan())
     assert torch.equal(out[want.isinf()].double(), want[want.isinf()])
+
+
+@pytest.mark.parametrize("m,n,k", [(40, 72, 64), (600, 520, 512), (1100, 1100, 96), (3000, 2304, 768)])
+@pytest.mark.parametrize("terms", [1, 2, 5])
+def test_fp32_sums_of_few_terms(m, n, k, terms):
+    """A row with few non-zero values is as exact as fp32 products: each of its T terms is off by
+    at most 2^-24 of it (and the partial sums of the smaller pieces by 2^-27 of it), as is each
+    of the T additions, half of it on average."""
+    from systems_for_llms_amd import _lib
+
+    a, w = operands(m, n, k, torch.float32)
+    g = torch.Generator(device="cuda").manual_seed(9)
+    keep = torch.zeros_like(a).scatter_(1, torch.rand(a.shape, device="cuda", generator=g).argsort(1)[:, :terms], 1.0)
+    a = a * keep
+    out = torch.full((m, n), float("nan"), device="cuda")
+    _lib.call("sfl_gemm", a.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k, 0, 0, 0, _lib.stream_handle())
+    wd = w.double().t().contiguous()
+    error, size = out.double() - a.double() @ wd, a.double().abs() @ wd.abs()
+    assert (error.abs() <= size * ((2 * terms - 1) * 1.125 * 2.0 ** -24)).all()
+    # Uniform mantissas round by 2^-25 sqrt(2/3) rms or less, and to either side.
+    relative = error / size
+    assert relative.square().mean().sqrt().item() <= (2 * terms - 1) ** 0.5 * 2.0 ** -25
+    assert (relative * torch.sign(out)).mean().abs().item() <= 2.0 ** -29
+
+
+@pytest.mark.parametrize("m,n,k", [(40, 72, 64), (300, 1040, 96), (1100, 1100, 64)])
+def test_fp32_operands_near_the_smallest(m, n, k):
+    """Operands whose 24 bits reach below the smallest bf16 subnormal keep all of them."""
+    from systems_for_llms_amd import _lib
+
+    a, w = operands(m, n, k, torch.float32)
+    a[1::2] *= 2.0 ** torch.randint(-124, -108, (m // 2, 1), device="cuda").float()
+    w = w * 2.0 ** 30
+    out = torch.full((m, n), float("nan"), device="cuda")
+    _lib.call("sfl_gemm", a.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k, 0, 0, 0, _lib.stream_handle())
+    want, bound = exact(a, w)
+    assert ((out.double() - want).abs() <= bound).all()
 
 
 def test_part_size_is_checked():
