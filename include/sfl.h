@@ -128,6 +128,11 @@ int sfl_decode_attention_out_proj(const float* q, const void* k, const void* v,
                                   int heads, int capacity, int head_dim, float scale, int dtype,
                                   void* stream);
 
+/* How many workgroups sfl_decode_attention_out_proj launches per (batch, head):
+ * each attends to the whole row and projects a part of the outputs. 1, 2 or 4
+ * by the sizes alone (0: bad arguments). */
+int sfl_decode_out_proj_workgroups(int batch, int heads, int capacity, int head_dim, int dtype);
+
 
 /* ---- decode step of the llmlab decoder (model dtype F32, BF16 or F16) -----
  * One step processes one token per sequence for `batch` <= 65536 sequences.

@@ -27,6 +27,7 @@ SIGNATURES: dict[str, list] = {
     "sfl_decode_attention_static": [P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int,
                                     c_int, c_int, P],
     "sfl_decode_attention_static_scratch_bytes": [],
+    "sfl_decode_out_proj_workgroups": [c_int, c_int, c_int, c_int, c_int],
     "sfl_decode_attention_out_proj": [P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_float, c_int, P],
     "sfl_packed_gemv_elems": [c_int, c_int],
     "sfl_pack_gemv_weights": [P, P, c_int, c_int, c_int, P],

@@ -747,21 +747,34 @@ inline bool gqa_mfma_fits(const DecodeCall& c) {
 // log2 of the workgroups that share one head's output projection. A short batch
 // has a workgroup (of the whole chip's 256 CUs) per head, which pulls the head's
 // d_model columns of W_o through one CU beside its keys: with 2 or 4 workgroups
-// that each attend to the whole row (its second reader finds the row in L2 or
-// the MALL) and project a part of the outputs, the launch is shorter as long as
-// each still has a CU of its own, longer beyond. us at 1 / 2 / 4 / 8 workgroups
-// (bf16, D 64, weights and caches from HBM):
-//   batch 1, 16 heads, 611 keys   8.7 /  8.0 /  7.6 /  7.6
-//   batch 1, 16 heads, 3583 keys 22.9 / 21.3 / 20.3 / 19.6
-//   batch 1, 12 heads, 611 keys   8.2 /  8.2 /  7.8 /  7.8 (fp16)
-//   batch 4, 16 heads, 500 keys   8.7 /  8.0 /  7.8 / 12.4 (8: 512 workgroups)
-//   batch 8, 16 heads, 3583 keys 27.1 / 27.0 / 52.7 (4: 512 workgroups)
-// A wave keeps at least half a tile of the projection.
-inline int proj_share_log2(long groups, int waves, int tiles) {
+// that each attend to the whole row and project a part of the outputs, the
+// launch is shorter as long as each still has a CU of its own and the rows that
+// are read 2 or 4 times come from a cache. The workgroups of a head are
+// blocks x, x + groups, ...: with groups a multiple of 8 they sit on one XCD and
+// share its L2, which pays while all they read fits the 256 MB of the MALL; with
+// other counts the rows come from the MALL, 2 workgroups gain nothing and 4
+// only on small caches (up to 12 MB). us at 1 / 2 / 4 workgroups (bf16, weights
+// and caches from HBM; groups = batch * heads, rows full; * the choice):
+//   16 groups D 64   3.6K keys 22.7 / 21.1 / 20.2*   16K 78.9 / 75.0 / 72.2*   65K 295* / 288 / 287
+//   32 groups D 128  4K        75.8 / 57.5 / 47.6*    8K 111 / 92.4* / 82.5
+//   48 groups D 64   1K        11.0 / 10.5 / 10.1*    8K 44.9 / 44.0* / 44.9   16K 82.5* / 82.0 / 84.1
+//   64 groups D 64   500       8.4 / 7.6 / 7.3*       8K 46.8 / 46.9* / 51.2   65K 329* / 355 / 465
+//   128 groups D 64  500       8.7 / 7.9* / 13.9      4K 26.4 / 26.4* / 51     16K 95.2* / 111 / 230
+//   12 groups D 64   611       8.2 / 8.2 / 7.8*       4K 24.2 / 25.1 / 23.9*   16K 77.7* / 80.7 / 78.5
+//   36 groups D 64   1K        11.0 / 11.4 / 10.8*    4K 25.2* / 27.2 / 26.7
+//   60 groups D 64   1K        11.2* / 11.8 / 11.4    6 groups 4K 22.9* / 24.1 / 25.5
+// (8 workgroups gain no more than 4.) At least half the waves get a tile of the
+// projection: with fewer, the launch only reads its rows more often.
+inline int proj_share_log2(long groups, long cache_bytes, int waves, int tiles) {
+  const auto fits = [&](int s) { return (groups << s) <= 256 && (waves << s) <= 2 * tiles; };
+  if (groups % kXcds) return fits(2) && cache_bytes <= (12L << 20) ? 2 : 0;
   int share = 0;
-  while (share < 2 && (groups << (share + 1)) <= 256 && (waves << (share + 1)) <= 2 * tiles) ++share;
+  while (share < 2 && fits(share + 1) && (cache_bytes << (share + 1)) <= (256L << 20)) ++share;
   return share;
 }
+
+// K and V of a launch, in bytes.
+inline long kv_bytes(long groups, int cap, int dim, int elem_bytes) { return 2 * groups * cap * dim * elem_bytes; }
 
 template <typename T, typename TQ, typename TO, int D, int G>
 int launch_attn(const DecodeCall& c) {
@@ -781,7 +794,7 @@ int launch_attn(const DecodeCall& c) {
   const long groups = long(c.batch) * c.kv_heads * c.splits;
   int splits = c.splits, share = 0;
   if constexpr (std::is_same<TO, resid_t>::value) {
-    share = proj_share_log2(groups, W, c.d_model / 16);
+    share = proj_share_log2(groups, kv_bytes(groups, c.cap, D, Elem<T>::bytes), W, c.d_model / 16);
     splits = share;
   }
   hipLaunchKernelGGL((decode_attn_kernel<T, TQ, TO, D, G, W>), dim3(unsigned(groups), 1u << share),
@@ -882,6 +895,15 @@ extern "C" int sfl_decode_attention_out_proj(const float* q, const void* k, cons
   if (dtype == SFL_DTYPE_BF16) return proj_dims<bf16_t>(c);
   if (dtype == SFL_DTYPE_F16) return proj_dims<f16_t>(c);
   return proj_dims<float>(c);
+}
+
+extern "C" int sfl_decode_out_proj_workgroups(int batch, int heads, int capacity, int head_dim, int dtype) {
+  using namespace sfl;
+  const int elem_bytes = dtype == SFL_DTYPE_F32 ? 4 : dtype == SFL_DTYPE_BF16 || dtype == SFL_DTYPE_F16 ? 2 : 0;
+  if (batch < 1 || heads < 1 || capacity < 1 || head_dim < 16 || head_dim > 128 || !elem_bytes) return 0;
+  const long groups = long(batch) * heads;
+  const int waves = head_dim <= 64 ? waves_for<float, 64, 1>() : waves_for<float, 128, 1>();
+  return 1 << proj_share_log2(groups, kv_bytes(groups, capacity, head_dim, elem_bytes), waves, heads * head_dim / 16);
 }
 
 namespace {

@@ -109,3 +109,19 @@ def test_prefill_layers_rejects_before_any_launch():
         args = _lib.PrefillArgs(**{**sizes, **pointers, **change})
         assert _lib.lib().sfl_prefill_layers(ctypes.addressof(args), None) != 0, change
         assert "prefill_layers" in _lib.lib().sfl_last_error().decode()
+
+
+def test_output_projection_is_shared_only_while_the_rows_stay_cached():
+    """Workgroups per head by (batch, heads, capacity, head dim, dtype): every head's K and V is
+    read by each, so long caches, and heads whose workgroups sit on several XCDs, keep one."""
+    from systems_for_llms_amd import _lib
+
+    count = _lib.lib().sfl_decode_out_proj_workgroups
+    bf16, f32 = 1, 0
+    for args, want in (((1, 16, 4096, 64, bf16), 4), ((4, 16, 4096, 64, bf16), 4), ((4, 16, 8192, 64, bf16), 2),
+                       ((4, 16, 16384, 64, bf16), 1), ((4, 16, 65536, 64, bf16), 1), ((8, 16, 4096, 64, bf16), 2),
+                       ((8, 16, 4096, 64, f32), 1), ((8, 16, 16384, 64, bf16), 1), ((16, 16, 256, 64, bf16), 1),
+                       ((1, 12, 1024, 64, bf16), 4), ((1, 12, 4096, 64, bf16), 4), ((1, 12, 8192, 64, bf16), 1),
+                       ((10, 12, 1024, 64, bf16), 2), ((9, 12, 1024, 64, bf16), 1), ((1, 6, 1024, 64, bf16), 1),
+                       ((1, 4, 64, 16, f32), 1), ((0, 4, 64, 64, bf16), 0), ((1, 4, 64, 64, 7), 0)):
+        assert count(*args) == want, args

@@ -112,11 +112,12 @@ def test_attention_out_proj_matches_reference(dtype, dim, batch, heads):
         torch.testing.assert_close(got[1], x0[1].double(), atol=0, rtol=0)
 
 
-# Workgroups per head's projection: 4 with more of them than tiles (48 tiles, 64 waves), 4 at the limit of
-# 256 workgroups, 2, and 2 of 8 waves.
+# Workgroups per head's projection: 4 with more of their waves than tiles (48 tiles, 64 waves), 4 at the limit
+# of 256 workgroups, 1 and 2 at more than half of them, 1 and 2 of 8 waves, 4 on several XCDs.
 @pytest.mark.parametrize("dtype,dim,batch,heads", [(torch.float16, 64, 1, 12), (torch.bfloat16, 64, 4, 16),
                                                    (torch.bfloat16, 32, 5, 20), (torch.float32, 64, 8, 16),
-                                                   (torch.bfloat16, 128, 11, 9)])
+                                                   (torch.bfloat16, 128, 11, 9),
+                                                   (torch.bfloat16, 128, 8, 12), (torch.float16, 64, 3, 12)])
 def test_attention_out_proj_shared_by_workgroups(dtype, dim, batch, heads):
     test_attention_out_proj_matches_reference(dtype, dim, batch, heads)
 
