@@ -72,20 +72,67 @@ int launch_begin(const sfl_prefill_args* p, hipStream_t s) {
 }  // namespace
 }  // namespace sfl
 
-extern "C" int sfl_prefill_layers(const sfl_prefill_args* p, void* stream) {
-  const char* what = "prefill_layers";
-  if (!p || !p->given || !p->tokens || !p->predicted || !p->prompt_len || !p->pos || !p->lengths || !p->x_last || !p->emb || !p->attn_norm || !p->w_qkv || !p->w_out || !p->ffn_norm || !p->w13 || !p->w2 ||
-      !p->k_cache || !p->v_cache || !p->x || !p->act || !p->q || !p->attn || !p->hidden ||
+namespace sfl {
+namespace {
+
+// Whatever an entry point of the sequence would refuse, refused before the
+// first launch: a call that fails leaves the session as it was.
+int check_prefill(const sfl_prefill_args* p, const char* what) {
+  if (!p || !p->given || !p->tokens || !p->predicted || !p->prompt_len || !p->pos || !p->lengths || !p->x_last ||
+      !p->emb || !p->attn_norm || !p->w_qkv || !p->w_out || !p->ffn_norm || !p->w13 || !p->w2 || !p->k_cache ||
+      !p->v_cache || !p->cos_t || !p->sin_t || !p->x || !p->act || !p->q || !p->attn || !p->hidden ||
       (p->fold && (!p->ss || !p->rscale)))
     return set_error(SFL_ERR_INVALID, "%s: null pointer argument", what);
   if (p->layers < 1 || p->batch < 1 || p->seq < 1 || p->d_model < 1 || p->heads < 1 || p->d_ff < 1 ||
-      p->d_model % p->heads || p->d_model % 16 || p->given_len < p->seq || p->capacity < p->given_len || long(p->batch) * p->seq > (1L << 31) - 1)
+      p->d_model % p->heads || p->d_model % 16 || p->given_len < p->seq || p->capacity < p->given_len ||
+      long(p->batch) * p->seq > (1L << 31) - 1)
     return set_error(SFL_ERR_INVALID, "%s: bad sizes", what);
-  const auto off16 = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 != 0; };
-  if (off16(p->x) || off16(p->x_last))
-    return set_error(SFL_ERR_INVALID, "%s: x and x_last must be 16-byte aligned", what);
   if (p->dtype != SFL_DTYPE_F32 && p->dtype != SFL_DTYPE_BF16 && p->dtype != SFL_DTYPE_F16)
     return set_error(SFL_ERR_UNSUPPORTED, "%s: model dtype must be F32, BF16 or F16", what);
+  if (!(p->scale > 0.f) || !__builtin_isfinite(p->scale))
+    return set_error(SFL_ERR_INVALID, "%s: scale must be finite and positive", what);
+  const bool f32 = p->dtype == SFL_DTYPE_F32;
+  const long m = long(p->batch) * p->seq, d = p->d_model, f = p->d_ff, dk = d / p->heads;
+  if (dk != 32 && dk != 64 && dk != 128 && !(f32 && dk == 16))
+    return set_error(SFL_ERR_UNSUPPORTED, "%s: head dim must be 32, 64 or 128 (F32: or 16)", what);
+  if (f % 8) return set_error(SFL_ERR_UNSUPPORTED, "%s: d_ff must be a multiple of 8", what);
+  if ((p->seq + 63L) / 64 * p->batch * p->heads > (1L << 31) - 1)
+    return set_error(SFL_ERR_UNSUPPORTED, "%s: too many query tiles", what);
+  // [m, k] x [n, k]^T: 32-bit operand offsets, or the kernel for any size with its grid of up to 65535 token tiles.
+  const auto gemm_ok = [&](long n, long k) {
+    const long limit = f32 ? 1L << 29 : 1L << 30;
+    return (k % (f32 ? 32 : 64) == 0 && m * k < limit && n * k < limit) || m <= 65535L * (f32 ? 64 : 128);
+  };
+  if (!gemm_ok(3 * d, d) || !gemm_ok(d, d) || !gemm_ok(2 * f, d) || !gemm_ok(d, f))
+    return set_error(SFL_ERR_UNSUPPORTED, "%s: too many rows", what);
+  if (p->fold && (f32 || d % 64 || f % 64 || d > 2048 || m * d >= 1L << 30 || m * f >= 1L << 30 ||
+                  3 * d * d >= 1L << 30 || 2 * f * d >= 1L << 30))
+    return set_error(SFL_ERR_UNSUPPORTED, "%s: folded norms need 16-bit weights, d_model and d_ff multiples of 64, "
+                     "d_model at most 2048 and operands under 2^30 elements", what);
+  const auto off = [](const void* q, unsigned n) { return reinterpret_cast<uintptr_t>(q) % n != 0; };
+  bool bad = off(p->x, 16) || off(p->x_last, 16) || (p->fold && off(p->act, 8));
+  if (f32) bad = bad || off(p->act, 16) || off(p->q, 16) || off(p->attn, 16) || off(p->hidden, 16);
+  for (int l = 0; l < p->layers; ++l) {
+    if (!p->attn_norm[l] || !p->w_qkv[l] || !p->w_out[l] || !p->ffn_norm[l] || !p->w13[l] || !p->w2[l] ||
+        !p->k_cache[l] || !p->v_cache[l])
+      return set_error(SFL_ERR_INVALID, "%s: null pointer argument (layer %d)", what, l);
+    if (p->fold) bad = bad || off(p->ffn_norm[l], 8) || (l > 0 && off(p->attn_norm[l], 8));
+    if (f32)
+      bad = bad || off(p->w_qkv[l], 16) || off(p->w_out[l], 16) || off(p->w13[l], 16) || off(p->w2[l], 16) ||
+            off(p->k_cache[l], 16) || off(p->v_cache[l], 16);
+  }
+  if (bad)
+    return set_error(SFL_ERR_INVALID, "%s: x and x_last must be 16-byte aligned, folded norms' act and gains 8-byte, "
+                     "F32 operands and outputs 16-byte", what);
+  return SFL_OK;
+}
+
+}  // namespace
+}  // namespace sfl
+
+extern "C" int sfl_prefill_layers(const sfl_prefill_args* p, void* stream) {
+  const char* what = "prefill_layers";
+  if (int rc = check_prefill(p, what)) return rc;
   const hipStream_t s = static_cast<hipStream_t>(stream);
   const int m = p->batch * p->seq, t = p->seq, d = p->d_model, f = p->d_ff, h = p->heads, dk = d / h, dt = p->dtype;
   const int F32 = SFL_DTYPE_F32;
@@ -95,11 +142,13 @@ extern "C" int sfl_prefill_layers(const sfl_prefill_args* p, void* stream) {
   const long os[3] = {long(t) * h * dk, dk, long(h) * dk};
   const int part_o = sfl_gemm_norm_part(m, d, d), part_f = sfl_gemm_norm_part(m, d, f);
   const int parts_o = (d + part_o - 1) / part_o, parts_f = (d + part_f - 1) / part_f;
-#define SFL_TRY(call)           \
-  do {                          \
+#define SFL_TRY(call)               \
+  do {                              \
     if (int rc = (call)) return rc; \
   } while (0)
-  SFL_TRY(dt == F32 ? launch_begin<float>(p, s) : dt == SFL_DTYPE_BF16 ? launch_begin<bf16_t>(p, s) : launch_begin<f16_t>(p, s));
+  SFL_TRY(dt == F32              ? launch_begin<float>(p, s)
+          : dt == SFL_DTYPE_BF16 ? launch_begin<bf16_t>(p, s)
+                                 : launch_begin<f16_t>(p, s));
   if (p->fold)
     SFL_TRY(sfl_rmsnorm_rows_scaled(p->x, p->attn_norm[0], p->act, p->rscale, m, d, dt, stream));
   for (int l = 0; l < p->layers; ++l) {

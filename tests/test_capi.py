@@ -6,6 +6,7 @@ from pathlib import Path
 import pytest
 
 ROOT = Path(__file__).resolve().parents[1]
+INVALID, UNSUPPORTED = -1, -2  # SFL_ERR_*
 
 
 def declared_symbols():
@@ -109,6 +110,32 @@ def test_prefill_layers_rejects_before_any_launch():
         args = _lib.PrefillArgs(**{**sizes, **pointers, **change})
         assert _lib.lib().sfl_prefill_layers(ctypes.addressof(args), None) != 0, change
         assert "prefill_layers" in _lib.lib().sfl_last_error().decode()
+
+
+def test_prefill_layers_refuses_what_its_layers_would_before_any_launch():
+    """Argument errors (-1, -2), not the failed launch (-3) a call without a GPU ends with."""
+    import ctypes
+
+    from systems_for_llms_amd import _lib
+
+    sizes = dict(dtype=2, layers=2, batch=1, seq=4, given_len=4, d_model=64, heads=2, d_ff=64, capacity=4, fold=0,
+                 scale=1.0)
+    pointers = {name: 16 if kind is _lib.P else (_lib.P * 2)(16, 16) for name, kind in _lib.PrefillArgs._fields_
+                if name not in sizes}
+    second, odd = (lambda: (_lib.P * 2)(16, None)), (lambda: (_lib.P * 2)(16, 20))
+    fold, f32 = dict(fold=1), dict(dtype=0)
+    for change, code in ((dict(fold, dtype=0), UNSUPPORTED), (dict(fold, d_ff=96), UNSUPPORTED),
+                         (dict(fold, d_model=96, heads=3), UNSUPPORTED),
+                         (dict(fold, d_model=4096, heads=32), UNSUPPORTED), (dict(fold, ffn_norm=odd()), INVALID),
+                         (dict(fold, attn_norm=odd()), INVALID), (dict(fold, act=20), INVALID),
+                         (dict(d_model=96), UNSUPPORTED), (dict(heads=4), UNSUPPORTED), (dict(d_ff=60), UNSUPPORTED),
+                         (dict(cos_t=None), INVALID), (dict(sin_t=None), INVALID), (dict(scale=0.0), INVALID),
+                         (dict(scale=float("nan")), INVALID), (dict(f32, act=24), INVALID), (dict(f32, w2=odd()), INVALID),
+                         (dict(f32, batch=1 << 22, seq=2, d_model=48, heads=3), UNSUPPORTED),
+                         *((dict({name: second()}), INVALID) for name in ("attn_norm", "w_qkv", "w_out", "ffn_norm",
+                                                                         "w13", "w2", "k_cache", "v_cache"))):
+        args = _lib.PrefillArgs(**{**sizes, **pointers, **change})
+        assert _lib.lib().sfl_prefill_layers(ctypes.addressof(args), None) == code, change
 
 
 def test_output_projection_is_shared_only_while_the_rows_stay_cached():
