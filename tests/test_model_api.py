@@ -145,3 +145,55 @@ def test_parameter_version_sees_changes_and_ends_on_cyclic_modules():
     with torch.no_grad():
         model.layers[1].ffn.w2.weight.mul_(2)
     assert parameter_version(model) != first
+
+
+class _Wrapped(torch.nn.Module):
+    """A module in front of another, as ``torch.compile`` makes it."""
+
+    def __init__(self, inner):
+        super().__init__()
+        self.inner = inner
+
+    def __getattr__(self, name):
+        return super().__getattr__(name) if name == "inner" else getattr(self.inner, name)
+
+
+def _rearranged(model):
+    """Layer 0 wrapped, its projection a plain object's; layer 1's feed-forward part behind a property."""
+    from types import SimpleNamespace
+
+    block, plain = model.layers[0], model.layers[0].attn.output_proj
+    del block.attn.output_proj
+    object.__setattr__(block.attn, "output_proj", SimpleNamespace(weight=plain.weight))
+    model.layers[0] = _Wrapped(block)
+    block = model.layers[1]
+    inner = block.ffn
+    del block.ffn
+    block.__class__ = type("Behind", (type(block),), {"ffn": property(lambda self: inner)})
+    return model
+
+
+def test_layer_weights_are_found_wherever_attributes_find_them():
+    from systems_for_llms_amd.engine import _layer_weights
+
+    cfg = ModelConfig(vocab_size=50, context_length=8, d_model=32, num_layers=2, num_heads=2, d_ff=64)
+    model = TransformerLM.from_config(cfg, device="cpu", dtype=torch.float32)
+    plain = [[w.data_ptr() for w in weights] for weights in _layer_weights(model)]
+    assert plain == [[blk.attn_norm.weight.data_ptr() for blk in model.layers],
+                     [blk.attn.output_proj.weight.data_ptr() for blk in model.layers],
+                     [blk.ffn_norm.weight.data_ptr() for blk in model.layers],
+                     [blk.ffn.w2.weight.data_ptr() for blk in model.layers]]
+    assert [[w.data_ptr() for w in weights] for weights in _layer_weights(_rearranged(model))] == plain
+
+
+@pytest.mark.gpu
+def test_prefill_of_wrapped_blocks():
+    from systems_for_llms_amd.engine import DecodeSession
+
+    cfg = ModelConfig(vocab_size=50, context_length=16, d_model=64, num_layers=2, num_heads=2, d_ff=64)
+    model = TransformerLM.from_config(cfg, device="cuda", dtype=torch.bfloat16)
+    model.load_state_dict(seeded_state_dict(cfg, 4))
+    ids = torch.arange(12, device="cuda").view(1, 12)
+    want = DecodeSession(model, 1).prefill(ids, all_logits=True)
+    got = DecodeSession(_rearranged(model), 1).prefill(ids, all_logits=True)
+    assert torch.equal(got, want)
