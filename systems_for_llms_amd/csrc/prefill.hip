@@ -2,6 +2,8 @@
 // tokens is 5 launches of 5-13 us per layer; issued one ctypes call at a time
 // they cost the host 7-25 us each, so the 100M model's short prompts waited on
 // Python (forward of 2 x 205 tokens: 830 us of host time, ~450 of kernels).
+#include <algorithm>
+
 #include "common.hpp"
 
 using namespace sfl;
@@ -9,9 +11,10 @@ using namespace sfl;
 namespace sfl {
 namespace {
 
-// State of the session and embedding of the prompt: x[m] = emb[given[m]] in
-// fp32, one workgroup per prompt position; the [batch, capacity] token arrays
-// are dealt over the whole grid. Bound by the launch (5 us for 2048 rows of
+// State of the session and embedding of the prompt: x[r] = emb[given[r]] in
+// fp32, one workgroup per prompt position r < rows; the [batch, capacity] token
+// arrays are dealt over the whole grid, which has workgroups of its own for
+// them where the prompt is short and the capacity long (begin_grid). Bound by the launch (5 us for 2048 rows of
 // 512): one kernel where fills, copies and the gather were six, each 1.5-5 us
 // with 10-25 us of host time ahead of the first layer. Every prefill is ~25 us
 // shorter for this and the last position's kernel below: 24 tokens of 3
@@ -22,21 +25,23 @@ __global__ __launch_bounds__(128) void prefill_begin_kernel(
     int batch, int cap, int64_t* __restrict__ tokens, int64_t* __restrict__ predicted, int32_t* __restrict__ prompt_len) {
   constexpr int V = vec_elems<T>();
   const unsigned m = blockIdx.x;
-  const unsigned b = m / unsigned(seq), t = m - b * unsigned(seq);
-  const T* src = emb + given[long(b) * given_len + t] * d;
-  float* xr = x + long(m) * d;
-  const bool wide = reinterpret_cast<uintptr_t>(emb) % 16 == 0;  // rows are multiples of 32 bytes
-  for (int i = V * threadIdx.x; i < d; i += V * 128) {
-    float v[V];
-    if (wide) {
-      unpack16<T>(load16(src + i), v);
-    } else {
+  if (m < unsigned(batch) * unsigned(seq)) {
+    const unsigned b = m / unsigned(seq), t = m - b * unsigned(seq);
+    const T* src = emb + given[long(b) * given_len + t] * d;
+    float* xr = x + long(m) * d;
+    const bool wide = reinterpret_cast<uintptr_t>(emb) % 16 == 0;  // rows are multiples of 32 bytes
+    for (int i = V * threadIdx.x; i < d; i += V * 128) {
+      float v[V];
+      if (wide) {
+        unpack16<T>(load16(src + i), v);
+      } else {
 #pragma unroll
-      for (int j = 0; j < V; ++j) v[j] = load_scalar<T>(src + i + j);
+        for (int j = 0; j < V; ++j) v[j] = load_scalar<T>(src + i + j);
+      }
+#pragma unroll
+      for (int j = 0; j < V; j += 4)
+        *reinterpret_cast<float4*>(xr + i + j) = make_float4(v[j], v[j + 1], v[j + 2], v[j + 3]);
     }
-#pragma unroll
-    for (int j = 0; j < V; j += 4)
-      *reinterpret_cast<float4*>(xr + i + j) = make_float4(v[j], v[j + 1], v[j + 2], v[j + 3]);
   }
   const long all = long(batch) * cap;
   for (long i = long(m) * 128 + threadIdx.x; i < all; i += long(gridDim.x) * 128) {
@@ -61,9 +66,18 @@ __global__ __launch_bounds__(256) void prefill_end_kernel(const float* __restric
   }
 }
 
+// Workgroups of prefill_begin_kernel: one per prompt position, and enough that
+// a thread fills about 4 entries of the token arrays (up to 8 per CU; with the
+// prompt's alone, one token at a capacity of 131072 filled them on one CU:
+// 174 us, now 4.7; 4096 7.2 -> 4.6).
+inline unsigned begin_grid(long rows, long entries) {
+  return unsigned(std::max(rows, std::min(2048L, (entries + 511) / 512)));
+}
+
 template <typename T>
 int launch_begin(const sfl_prefill_args* p, hipStream_t s) {
-  hipLaunchKernelGGL(prefill_begin_kernel<T>, dim3(unsigned(p->batch) * unsigned(p->seq)), dim3(128), 0, s, p->given,
+  const dim3 grid(begin_grid(long(p->batch) * p->seq, long(p->batch) * p->capacity));
+  hipLaunchKernelGGL(prefill_begin_kernel<T>, grid, dim3(128), 0, s, p->given,
                      static_cast<const T*>(p->emb), p->x, p->d_model, p->seq, p->given_len, p->batch, p->capacity,
                      p->tokens, p->predicted, p->prompt_len);
   return check_launch("prefill_layers");

@@ -703,12 +703,12 @@ def test_f32_forward_is_one_prefill_pass_equal_to_the_oracle():
 
 
 @pytest.mark.parametrize("batch,t,given,cap,offset", [(1, 1, 1, 1, 0), (3, 5, 5, 40, 0), (2, 7, 11, 11, 0), (5, 3, 4, 33, 0),
-                                                    (4, 6, 6, 6, 1)])
+                                                    (4, 6, 6, 6, 1), (2, 1, 3, 3000, 0), (1, 700, 701, 1500, 0)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_prefill_loads_the_session_state(batch, t, given, cap, offset, dtype):
     """Tokens, predictions and counters after a prefill into a used session, and the embedded
     prompt (through the logits), also from an embedding table off a 16-byte boundary."""
-    cfg = ModelConfig(vocab_size=97, context_length=64, d_model=64, num_layers=1, num_heads=2, d_ff=96)
+    cfg = ModelConfig(vocab_size=97, context_length=max(64, cap), d_model=64, num_layers=1, num_heads=2, d_ff=96)
     model = gpu_model(cfg, seeded_state_dict(cfg, 3), dtype)
     ids = torch.randint(0, 97, (batch, given), generator=torch.Generator().manual_seed(t))
     plain = DecodeSession(model, batch, cap).prefill(ids[:, :t], all_logits=True)
