@@ -232,12 +232,8 @@ def attention(q, k, v, schedule, spec, document_ids=None, num_warps=4, num_stage
 
 
 def _launch_masked(q, k, v, out, lse, *rest):
-    """``torch.ops.sfl.masked_attention``, past the dispatcher where nothing watches it."""
-    if ops.launches_directly(q, k, v, out, lse):
-        ops.launch_masked_attention(q, k, v, out, lse, *rest)
-        ops.mark_written(out, lse)
-    else:
-        torch.ops.sfl.masked_attention(q, k, v, out, lse, *rest)
+    """``torch.ops.sfl.masked_attention``, without its autograd layers where nothing requires grad."""
+    ops.dispatch(torch.ops.sfl.masked_attention, (q, k, v, out, lse), (out, lse), *rest)
 
 
 def _record_launch_metadata(q, k, v, spec, implementation, destination):

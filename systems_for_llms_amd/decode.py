@@ -111,13 +111,9 @@ class PreparedDecode:
     variant: str
 
     def __call__(self) -> torch.Tensor:
-        args = (self.q, self.k, self.v, self.lengths, self.partial_max, self.partial_sum, self.partial_output,
-                self.output)
-        if ops.launches_directly(*args):
-            ops.launch_decode_attention(*args, self.splits, self.scale)
-            ops.mark_written(*args[4:])
-        else:
-            torch.ops.sfl.decode_attention(*args, self.splits, self.scale)
+        scratch = (self.partial_max, self.partial_sum, self.partial_output, self.output)
+        ops.dispatch(torch.ops.sfl.decode_attention, (self.q, self.k, self.v, self.lengths, *scratch), scratch,
+                     self.splits, self.scale)
         return self.output
 
     @property

@@ -43,30 +43,108 @@ def test_meta_and_fake_dispatch_launch_nothing():
         torch.ops.sfl.decode_attention(*_decode_args("cpu"))
 
 
-def test_direct_launches_only_where_nothing_watches_the_op():
-    from systems_for_llms_amd.ops import launches_directly
+def _prepared(*tensors):
+    from systems_for_llms_amd.decode import PreparedDecode
+
+    return PreparedDecode(*tensors, 3, 0.125, "token")
+
+
+def _masked(q):
+    from systems_for_llms_amd.attention import _launch_masked
+
+    out = torch.empty_like(q)
+    _launch_masked(q, q, q, out, None, 0.125, True, -1, -1, 0, None, None, None, None, True)
+    return out
+
+
+def _seen_by_mode(call):
     from torch.utils._python_dispatch import TorchDispatchMode
 
     class Watch(TorchDispatchMode):
         def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
             return func(*args, **(kwargs or {}))
 
-    seen, x = [], torch.zeros(2, 3)
-    assert launches_directly(x, None)
-    assert not launches_directly(x, x.clone().requires_grad_())
-    assert not launches_directly(torch.nn.Parameter(x, requires_grad=False))
+    seen = []
     with Watch():
-        seen.append(launches_directly(x))
-    with torch.overrides.BaseTorchFunctionMode():
-        seen.append(launches_directly(x))
-    with torch.autograd.forward_ad.dual_level():
-        seen.append(launches_directly(x))
-    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]):
-        seen.append(launches_directly(x))
-    torch.func.vmap(lambda row: (seen.append(launches_directly(x)), row)[1])(x)
-    torch.func.grad(lambda row: (seen.append(launches_directly(x)), row.sum())[1])(x)
-    torch.jit.trace(lambda row: (seen.append(launches_directly(row)), row + 1)[1], (x,), check_trace=False)
-    assert seen == [False] * 7 and launches_directly(x)
+        call()
+    return seen
+
+
+def _seen_by_function_mode(call):
+    class Watch(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    seen = []
+    with Watch():
+        call()
+    return seen
+
+
+def _seen_by_profiler(call):
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as profile:
+        call()
+    return [event.key.replace("::", ".") for event in profile.key_averages()]
+
+
+def _seen_by_observer(call):
+    import json
+    import tempfile
+    from pathlib import Path
+
+    with tempfile.TemporaryDirectory() as folder:
+        path = Path(folder) / "trace.json"
+        observer = torch.profiler.ExecutionTraceObserver()
+        observer.register_callback(str(path))
+        observer.start()
+        call()
+        observer.stop()
+        observer.unregister_callback()
+        return [node["name"].replace("::", ".") for node in json.loads(path.read_text())["nodes"]]
+
+
+def _seen_by_make_fx(call):
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    return [make_fx(lambda x: (call(), x)[1])(torch.zeros(1)).code]
+
+
+@pytest.mark.parametrize("watch", [_seen_by_mode, _seen_by_function_mode, _seen_by_profiler, _seen_by_observer,
+                                   _seen_by_make_fx])
+def test_operator_apis_launch_in_sight_of_whatever_watches(watch):
+    prepared = _prepared(*_decode_args("meta")[:8])
+    q = torch.empty(1, 2, 128, 64, device="meta", dtype=torch.bfloat16)
+    assert any("sfl.decode_attention" in name for name in watch(prepared))
+    assert any("sfl.masked_attention" in name for name in watch(lambda: _masked(q)))
+
+
+def test_operator_apis_are_traced_by_jit():
+    args = _decode_args("meta")[:8]
+    graph = torch.jit.trace(lambda *tensors: _prepared(*tensors)(), args, check_trace=False).graph
+    assert "sfl::decode_attention" in str(graph)
+    q = torch.empty(1, 2, 128, 64, device="meta", dtype=torch.bfloat16)
+    assert "sfl::masked_attention" in str(torch.jit.trace(_masked, (q,), check_trace=False).graph)
+
+
+def test_operator_apis_count_versions_and_leave_transforms_to_the_op(monkeypatch):
+    from systems_for_llms_amd import ops
+
+    tensors = _decode_args("meta")[:8]
+    args = tuple(t.clone() for t in tensors)
+    for guard in (ops._below_autograd, None):
+        monkeypatch.setattr(ops, "_below_autograd", guard)  # None: as in a torch without it
+        before = [t._version for t in args]
+        _prepared(*args)()
+        assert [t._version for t in args] == [v + (i >= 4) for i, v in enumerate(before)]
+        with torch.inference_mode():
+            _prepared(*[t.clone() for t in tensors])()  # inference tensors have no counter
+        with pytest.raises(RuntimeError, match="Batching rule not implemented"):
+            torch.func.vmap(lambda q: (_prepared(q, *args[1:])(), q)[1])(torch.stack([args[0]] * 2))
+        with pytest.raises(RuntimeError, match="functorch transforms"):
+            torch.func.grad(lambda q: (_prepared(q, *args[1:])(), q.sum())[1])(torch.zeros_like(args[0]))
+        torch.func.vmap(lambda row: (_prepared(*args)(), row)[1])(torch.zeros(2))
 
 
 def test_mark_written_bumps_versions_like_the_op():
@@ -90,6 +168,23 @@ def test_prepared_decode_bumps_the_output_version():
     op()
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         product.sum().backward()
+
+
+@pytest.mark.gpu
+def test_lazily_negated_tensors_are_resolved():
+    from systems_for_llms_amd.attention import attention, causal_prefill
+    from systems_for_llms_amd.decode import decode
+    from systems_for_llms_amd.masks import MaskSpec, compile_mask
+
+    g = torch.Generator(device="cuda").manual_seed(1)
+    k, v = (torch.randn((2, 2, 70, 64), device="cuda", generator=g).bfloat16() for _ in range(2))
+    q = torch.randn((2, 4, 64), device="cuda", generator=g).bfloat16()
+    assert torch.equal(decode(q, k, torch._neg_view(v)), decode(q, k, -v))
+    spec = MaskSpec(causal=True)
+    schedule = compile_mask(70, spec)
+    assert torch.equal(attention(torch._neg_view(k), k, v, schedule, spec), attention(-k, k, v, schedule, spec))
+    want, got = (torch.empty_like(k) for _ in range(2))
+    assert torch.equal(causal_prefill(k, torch._neg_view(k), v, got), causal_prefill(k, -k, v, want))
 
 
 @pytest.mark.gpu
