@@ -287,7 +287,8 @@ typedef struct {
 
 /*
  * The kernel sfl_masked_attention launches for this head dim, dtype, sequence
- * length and K/V row strides (elements), with its resource data. Replaces the
+ * length and K/V row strides (elements) without document labels, with its
+ * resource data. Replaces the
  * Triton CompiledKernel metadata the reference records when its caller passes
  * `launch_metadata` (attention_lab/triton_attention.py:39-57,
  * launch_metadata at :326-328). Needs a HIP device; launches nothing.
@@ -295,6 +296,11 @@ typedef struct {
 int sfl_masked_attention_kernel_info(int head_dim, int dtype, int n, long k_row_stride,
                                      long v_row_stride, int causal, int window_left,
                                      int window_right, int global_prefix, sfl_kernel_info* info);
+
+/* The same for a mask with document labels (kernels of their own at head dims 64 and 128). */
+int sfl_masked_attention_documents_kernel_info(int head_dim, int dtype, int n, long k_row_stride,
+                                               long v_row_stride, int causal, int window_left,
+                                               int window_right, int global_prefix, sfl_kernel_info* info);
 
 /* ---- prefill (weights in bf16, fp16 or fp32) ---------------------------------
  * C^T = W A^T on MFMAs; A [M, K] row-major (one row per token) and W [N, K]

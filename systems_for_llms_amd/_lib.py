@@ -21,6 +21,8 @@ DTYPE_F32X = 4    # fp32 values in the decode GEMVs' activation layout
 DTYPE_F16X2 = 5   # split-fp16 values in the decode GEMVs' activation layout
 
 P = c_void_p
+_INFO = [c_int, c_int, c_int, c_long, c_long, c_int, c_int, c_int, c_int, P]
+
 SIGNATURES: dict[str, list] = {
     "sfl_decode_attention": [P, P, P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int,
                              c_float, c_int, c_int, c_int, P],
@@ -42,7 +44,8 @@ SIGNATURES: dict[str, list] = {
                              POINTER(c_long), POINTER(c_long), c_float, c_int, c_int, c_int, c_int, P,
                              c_int, P, P, P, c_int, c_int, P],
     "sfl_masked_attention_block": [],
-    "sfl_masked_attention_kernel_info": [c_int, c_int, c_int, c_long, c_long, c_int, c_int, c_int, c_int, P],
+    "sfl_masked_attention_kernel_info": _INFO,
+    "sfl_masked_attention_documents_kernel_info": _INFO,
     "sfl_gemm": [P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, P],
     "sfl_gemm_qkv_rope": [P, P, c_int, c_int, c_int, c_int, P, P, P, P, P, c_int, c_int, P],
     "sfl_gemm_swiglu": [P, P, P, c_int, c_int, c_int, c_int, P],
@@ -132,11 +135,12 @@ def pack_gemv(w: torch.Tensor) -> torch.Tensor:
 
 def masked_kernel_info(head_dim: int, dtype: torch.dtype, n: int, k_row_stride: int,
                        v_row_stride: int, causal: bool = True, window_left: int = -1, window_right: int = -1,
-                       global_prefix: int = 0) -> KernelInfo:
+                       global_prefix: int = 0, documents: bool = False) -> KernelInfo:
     """Resource data of the kernel ``sfl_masked_attention`` launches for these shapes and mask
-    (windows < 0: unbounded)."""
+    (windows < 0: unbounded; ``documents``: with document labels)."""
     info = KernelInfo()
-    call("sfl_masked_attention_kernel_info", head_dim, dtype_code(dtype), n, k_row_stride, v_row_stride,
+    name = "sfl_masked_attention_documents_kernel_info" if documents else "sfl_masked_attention_kernel_info"
+    call(name, head_dim, dtype_code(dtype), n, k_row_stride, v_row_stride,
          int(causal), window_left, window_right, global_prefix, ctypes.addressof(info))
     return info
 

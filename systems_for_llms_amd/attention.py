@@ -242,7 +242,7 @@ def _record_launch_metadata(q, k, v, spec, implementation, destination):
     info = _lib.masked_kernel_info(
         q.shape[-1], q.dtype, q.shape[2], k.stride(2), v.stride(2), bool(spec.causal),
         -1 if spec.window_left is None else spec.window_left,
-        -1 if spec.window_right is None else spec.window_right, spec.global_prefix or 0)
+        -1 if spec.window_right is None else spec.window_right, spec.global_prefix or 0, spec.same_document)
     destination.update({
         "kernel_name": info.name.decode(),
         "n_regs": info.registers,

@@ -1110,13 +1110,15 @@ inline long row_keys(const MaskArgs& m, long n) {
 constexpr long kShortRowKeys = SFL_A32_SHORT_KEYS;
 
 template <typename T, int D, int NW>
-const void* attn32_fn(const MaskArgs& m) {
-  return m.docs ? reinterpret_cast<const void*>(&masked_attention32_kernel<T, D, NW, true>)
-                : reinterpret_cast<const void*>(&masked_attention32_kernel<T, D, NW, false>);
+MaskedLaunch attn32_launch(bool docs, const char* name, const char* name_docs) {
+  return {docs ? reinterpret_cast<const void*>(&masked_attention32_kernel<T, D, NW, true>)
+               : reinterpret_cast<const void*>(&masked_attention32_kernel<T, D, NW, false>),
+          docs ? name_docs : name, unsigned(NW / 2 * BQ), unsigned(NW * kWave)};
 }
 
+// docs: whether the mask has document labels (m.docs itself may be unknown).
 template <typename T>
-MaskedLaunch select_masked(int dim, long n, long k_row_stride, long v_row_stride, const MaskArgs& m) {
+MaskedLaunch select_masked(int dim, long n, long k_row_stride, long v_row_stride, const MaskArgs& m, bool docs) {
   const bool offsets32 = n * k_row_stride * 2 < (1L << 31) && n * v_row_stride * 2 < (1L << 31);
   const bool one_row = row_keys(m, n) <= kShortRowKeys;
   switch (dim) {
@@ -1125,17 +1127,17 @@ MaskedLaunch select_masked(int dim, long n, long k_row_stride, long v_row_stride
               unsigned(BQ), unsigned(kThreads)};
     case 64:
       if (offsets32 && one_row)
-        return {attn32_fn<T, 64, 2>(m),
-                "masked_attention32_kernel<D=64, 2 waves>", unsigned(BQ), unsigned(2 * kWave)};
+        return attn32_launch<T, 64, 2>(docs, "masked_attention32_kernel<D=64, 2 waves>",
+                                       "masked_attention32_kernel<D=64, 2 waves, documents>");
       if (offsets32)
-        return {attn32_fn<T, 64, kA32Waves>(m),
-                "masked_attention32_kernel<D=64>", unsigned(2 * BQ), unsigned(kA32Waves * kWave)};
+        return attn32_launch<T, 64, kA32Waves>(docs, "masked_attention32_kernel<D=64>",
+                                               "masked_attention32_kernel<D=64, documents>");
       return {reinterpret_cast<const void*>(&masked_attention_pair_kernel<T>), "masked_attention_pair_kernel<D=64>",
               unsigned(BQ), unsigned(kPairWaves * kWave)};
     case 128:  // (one row per workgroup at D = 128 needs 300 VGPRs: one wave per SIMD)
       if (offsets32)
-        return {attn32_fn<T, 128, kA32Waves>(m),
-                "masked_attention32_kernel<D=128>", unsigned(2 * BQ), unsigned(kA32Waves * kWave)};
+        return attn32_launch<T, 128, kA32Waves>(docs, "masked_attention32_kernel<D=128>",
+                                                "masked_attention32_kernel<D=128, documents>");
       return {reinterpret_cast<const void*>(&masked_attention_kernel<T, 128>), "masked_attention_kernel<D=128>",
               unsigned(BQ), unsigned(kThreads)};
     default: return {nullptr, nullptr, 0u, 0u};
@@ -1144,7 +1146,7 @@ MaskedLaunch select_masked(int dim, long n, long k_row_stride, long v_row_stride
 
 template <typename T>
 int launch_masked(AttnArgs a, int batch, int dim, hipStream_t stream) {
-  const MaskedLaunch l = select_masked<T>(dim, a.n, a.ks[2], a.vs[2], a.m);
+  const MaskedLaunch l = select_masked<T>(dim, a.n, a.ks[2], a.vs[2], a.m, a.m.docs != nullptr);
   if (!l.fn) return set_error(SFL_ERR_UNSUPPORTED, "masked_attention: head dim must be 32, 64 or 128");
   const dim3 grid(unsigned((a.n + l.queries_per_workgroup - 1) / l.queries_per_workgroup) *
                   unsigned(batch * a.heads));
@@ -1206,17 +1208,16 @@ extern "C" int sfl_masked_attention(const void* q, const void* k, const void* v,
 
 extern "C" int sfl_masked_attention_block(void) { return BQ; }
 
-extern "C" int sfl_masked_attention_kernel_info(int head_dim, int dtype, int n, long k_row_stride,
-                                                long v_row_stride, int causal, int window_left,
-                                                int window_right, int global_prefix, sfl_kernel_info* info) {
-  const char* what = "masked_attention_kernel_info";
+static int masked_kernel_info(const char* what, int head_dim, int dtype, int n, long k_row_stride, long v_row_stride,
+                              int causal, int window_left, int window_right, int global_prefix, bool docs,
+                              sfl_kernel_info* info) {
   if (!info) return set_error(SFL_ERR_INVALID, "%s: null pointer argument", what);
   if (n < 1 || k_row_stride < 0 || v_row_stride < 0 || global_prefix < 0)
     return set_error(SFL_ERR_INVALID, "%s: bad sizes", what);
   const MaskArgs m{causal, window_left, window_right, global_prefix, nullptr};
   MaskedLaunch l{};
-  if (dtype == SFL_DTYPE_BF16) l = select_masked<bf16_t>(head_dim, n, k_row_stride, v_row_stride, m);
-  else if (dtype == SFL_DTYPE_F16) l = select_masked<f16_t>(head_dim, n, k_row_stride, v_row_stride, m);
+  if (dtype == SFL_DTYPE_BF16) l = select_masked<bf16_t>(head_dim, n, k_row_stride, v_row_stride, m, docs);
+  else if (dtype == SFL_DTYPE_F16) l = select_masked<f16_t>(head_dim, n, k_row_stride, v_row_stride, m, docs);
   else return set_error(SFL_ERR_UNSUPPORTED, "%s: dtype must be BF16 or F16", what);
   if (!l.fn) return set_error(SFL_ERR_UNSUPPORTED, "%s: head dim must be 32, 64 or 128", what);
   hipFuncAttributes attr{};
@@ -1230,4 +1231,19 @@ extern "C" int sfl_masked_attention_kernel_info(int head_dim, int dtype, int n, 
   info->threads = int(l.threads);
   info->queries_per_workgroup = int(l.queries_per_workgroup);
   return SFL_OK;
+}
+
+extern "C" int sfl_masked_attention_kernel_info(int head_dim, int dtype, int n, long k_row_stride,
+                                                long v_row_stride, int causal, int window_left,
+                                                int window_right, int global_prefix, sfl_kernel_info* info) {
+  return masked_kernel_info("masked_attention_kernel_info", head_dim, dtype, n, k_row_stride, v_row_stride, causal,
+                            window_left, window_right, global_prefix, false, info);
+}
+
+extern "C" int sfl_masked_attention_documents_kernel_info(int head_dim, int dtype, int n, long k_row_stride,
+                                                          long v_row_stride, int causal, int window_left,
+                                                          int window_right, int global_prefix,
+                                                          sfl_kernel_info* info) {
+  return masked_kernel_info("masked_attention_documents_kernel_info", head_dim, dtype, n, k_row_stride, v_row_stride,
+                            causal, window_left, window_right, global_prefix, true, info);
 }

@@ -178,3 +178,21 @@ def test_launch_metadata_records_the_launched_kernels_resources(d):
         assert meta["shared_memory_bytes"] > 0 and meta["threads"] in (128, 256)
         assert meta["asm_sha256"] == {} and len(meta["library_sha256"]) == 64
         assert "not rocprof" in meta["source"]
+
+
+@pytest.mark.parametrize("d,n,name", [(32, 300, "masked_attention_kernel<D=32>"),
+                                      (64, 130, "masked_attention32_kernel<D=64, 2 waves, documents>"),
+                                      (64, 1000, "masked_attention32_kernel<D=64, documents>"),
+                                      (128, 300, "masked_attention32_kernel<D=128, documents>")])
+def test_launch_metadata_of_document_masks(d, n, name):
+    """Masks with documents run kernels of their own at head dims 64 and 128, which keep a tile's labels in LDS."""
+    q, k, v = (t.cuda() for t in inputs(1, 2, n, d, torch.bfloat16, 3))
+    plain, with_documents, docs = {}, {}, [i // 70 for i in range(n)]
+    spec = MaskSpec(causal=True)
+    attention(q, k, v, compile_mask(n, spec), spec, launch_metadata=plain)
+    spec = MaskSpec(causal=True, same_document=True)
+    attention(q, k, v, compile_mask(n, spec, document_ids=docs), spec, docs, launch_metadata=with_documents)
+    assert with_documents["kernel_name"] == name + " bf16"
+    labels = 0 if d == 32 else 8 * 64 * with_documents["threads"] // 64
+    assert with_documents["shared_memory_bytes"] >= plain["shared_memory_bytes"] + labels
+    assert (with_documents["kernel_name"] == plain["kernel_name"]) == (d == 32)
