@@ -658,6 +658,7 @@ __global__ __launch_bounds__(kGqaWaves * kWave) void decode_gqa32_kernel(
   for (int buf = 0; t0 < end; buf ^= 1) {
     const int tn = t0 + BT * W;
     if (tn < end) {
+      wait_lds_reads();  // of the tile before, whose buffer this refills
       issue(tn, buf ^ 1);
       __builtin_amdgcn_s_waitcnt(sfl_vmcnt(2 * NLD));  // this tile has landed, the next is in flight
     } else {

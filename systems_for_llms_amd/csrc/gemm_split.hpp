@@ -179,7 +179,10 @@ void gemm_split_kernel(typename SplitArgs<T>::type g) {
             for (int j = 0; j < NBM; ++j) acc[i][j] = mma_slot<T>(af[i], bf[j], acc[i][j]);
         }
       }
-      if (t + NS < mine) issue(st[wave][cur], wave + (t + NS) * NW);
+      if (t + NS < mine) {
+        wait_lds_reads();
+        issue(st[wave][cur], wave + (t + NS) * NW);
+      }
       cur = cur + 1 == NS ? 0 : cur + 1;
     }
   };

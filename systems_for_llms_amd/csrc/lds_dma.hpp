@@ -28,6 +28,11 @@ __device__ __forceinline__ unsigned lds_offset(const void* p) {
   return unsigned(size_t((__attribute__((address_space(3))) const char*)(p)));
 }
 
+// Waits for this wave's LDS reads: before lds_load16 refills what they read
+// without a barrier in between. (The compiler waits for a read where its value
+// is used, which may come after the refill is issued.)
+__device__ __forceinline__ void wait_lds_reads() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
 // s_waitcnt operand that waits for vmcnt <= n only (gfx9 encoding: vmcnt in
 // bits 3:0 and 15:14, expcnt 6:4 and lgkmcnt 11:8 left at their maxima).
 constexpr int sfl_vmcnt(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
