@@ -323,6 +323,13 @@ int sfl_masked_attention_documents_kernel_info(int head_dim, int dtype, int n, l
  * layers.py:114-115, transformer.py:137-138).
  */
 
+/* The output tile of an [m, k] x [n, k]^T product in 16-bit operands (k a
+ * multiple of 64, operands under 2^30 elements; n all the features: 3 d_model
+ * for q/k/v, 2 d_ff for SwiGLU): features x tokens of a workgroup, and whether
+ * its waves split K (each sums a share; the shares are added in wave order) or
+ * share it. epilogue: 0 sfl_gemm and the residual forms, 1 q/k/v, 2 SwiGLU. */
+int sfl_gemm_tile(int m, int n, int k, int epilogue, int* features, int* tokens, int* k_split);
+
 /* C = A W^T as fp32 (c_dtype F32; accumulate = 1 adds into C: the residual
  * update) or in the input type (c_dtype == dtype). */
 int sfl_gemm(const void* a, const void* w, void* c, int m, int n, int k, int dtype, int c_dtype,

@@ -53,6 +53,7 @@ SIGNATURES: dict[str, list] = {
     "sfl_rmsnorm_rows": [P, P, P, c_int, c_int, c_int, c_int, P],
     "sfl_rmsnorm_rows_scaled": [P, P, P, P, c_int, c_int, c_int, P],
     "sfl_gemm_residual_norm": [P, P, P, c_int, c_int, c_int, P, P, P, c_int, P],
+    "sfl_gemm_tile": [c_int, c_int, c_int, c_int, POINTER(c_int), POINTER(c_int), POINTER(c_int)],
     "sfl_gemm_norm_part": [c_int, c_int, c_int],
     "sfl_gemm_residual_norm_parts": [P, P, P, c_int, c_int, c_int, P, P, P, c_int, c_int, P],
     "sfl_norm_scale": [P, c_int, c_int, c_int, P, P],
@@ -156,6 +157,14 @@ def library_sha256() -> str:
 
         _LIB_SHA256 = hashlib.sha256(LIB_PATH.read_bytes()).hexdigest()
     return _LIB_SHA256
+
+
+def gemm_tile(m: int, n: int, k: int, epilogue: int = 0) -> tuple[int, int, bool]:
+    """Features and tokens of the tile a 16-bit GEMM of these sizes runs on, and whether its waves
+    split K (``sfl_gemm_tile``; epilogue 0 plain or residual, 1 q/k/v, 2 SwiGLU)."""
+    out = [c_int() for _ in range(3)]
+    call("sfl_gemm_tile", m, n, k, epilogue, *out)
+    return out[0].value, out[1].value, bool(out[2].value)
 
 
 def pointers(tensors):

@@ -661,6 +661,19 @@ extern "C" int sfl_gemm_residual_norm(const void* a, const void* w, float* x, in
   return gemm_residual_norm("gemm_residual_norm", a, w, x, m, n, k, gain_next, act_xg, ss_parts, 128, dtype, stream);
 }
 
+extern "C" int sfl_gemm_tile(int m, int n, int k, int epilogue, int* features, int* tokens, int* k_split) {
+  const char* what = "gemm_tile";
+  if (!features || !tokens || !k_split) return set_error(SFL_ERR_INVALID, "%s: null pointer argument", what);
+  if (m < 1 || n < 1 || k < 1 || epilogue < G_PLAIN || epilogue > G_SWIGLU)
+    return set_error(SFL_ERR_INVALID, "%s: bad sizes or epilogue", what);
+  if (!gemm32_path(m, n, k)) return set_error(SFL_ERR_UNSUPPORTED, "%s: K must be a multiple of %d", what, K2);
+  const Tile16 t = tile16_for(m, n, k, epilogue);
+  *features = t == S32x32 ? 32 : t <= S64x64 ? 64 : t <= T128x128 ? 128 : 256;
+  *tokens = t <= S64x32 ? 32 : t <= T128x64 ? 64 : t == T128x128 ? 128 : t == T256x256 ? 256 : 384;
+  *k_split = t <= S128x64;
+  return SFL_OK;
+}
+
 extern "C" int sfl_gemm_norm_part(int m, int n, int k) { return norm_part_of(tile16_for(m, n, k, G_PLAIN)); }
 
 extern "C" int sfl_gemm_residual_norm_parts(const void* a, const void* w, float* x, int m, int n, int k,

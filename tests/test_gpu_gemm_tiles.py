@@ -122,6 +122,53 @@ def test_normed_consumers(batch, seq, d, heads, d_ff, dtype):
     assert ((h[0].double() - want).abs() <= tol + (want.abs() + tol) * HALF_ULP[dtype] + 2.0 ** -25).all()
 
 
+# The tiles whose waves share K, with three and five K steps and ragged features and tokens: (features, tokens),
+# which the sizes must select.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tile,m,n,k", [((128, 64), 2049, 1028, 320), ((128, 128), 8278, 668, 192),
+                                        ((256, 256), 9151, 1076, 192), ((256, 384), 9345, 1688, 320)])
+def test_plain_and_residual_on_shared_k_tiles(tile, m, n, k, dtype):
+    from systems_for_llms_amd import _lib
+
+    assert _lib.gemm_tile(m, n, k) == (*tile, False)
+    test_plain_and_residual(m, n, k, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tile,batch,seq,d,heads,d_ff", [((128, 64), 5, 205, 768, 12, 2048),
+                                                         ((128, 128), 5, 1966, 192, 3, 344),
+                                                         ((256, 256), 17, 641, 384, 6, 536),
+                                                         ((256, 384), 31, 339, 576, 9, 840)])
+def test_normed_consumers_on_shared_k_tiles(tile, batch, seq, d, heads, d_ff, dtype):
+    from systems_for_llms_amd import _lib
+
+    assert _lib.gemm_tile(batch * seq, 3 * d, d, 1) == (*tile, False)
+    assert _lib.gemm_tile(batch * seq, 2 * d_ff, d, 2) == (*tile, False)
+    test_normed_consumers(batch, seq, d, heads, d_ff, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_rows_of_other_batches_agree_to_rounding(dtype):
+    """The order a row's products are added in depends on the tile, so on the rows beside it: equal
+    rows agree to twice the bound of any order, not bit for bit; in the same batch size they do."""
+    from systems_for_llms_amd import _lib
+
+    a, w = operands(9400, 1688, 1024, dtype)
+    want, bound = exact(a[:5], w)
+    st, code, outs, tiles = _lib.stream_handle(), _lib.dtype_code(dtype), [], set()
+    for m in (5, 301, 1300, 5000, 9400, 9400):
+        out = torch.full((m, 1688), float("nan"), device="cuda")
+        _lib.call("sfl_gemm", a.data_ptr(), w.data_ptr(), out.data_ptr(), m, 1688, 1024, code, 0, 0, st)
+        outs.append(out[:5])
+        if dtype != torch.float32:
+            tiles.add(_lib.gemm_tile(m, 1688, 1024))
+    assert dtype == torch.float32 or len(tiles) >= 4
+    for out in outs:
+        assert ((out.double() - want).abs() <= bound).all()
+        assert ((out.double() - outs[0].double()).abs() <= 2 * bound).all()
+    assert torch.equal(outs[-1], outs[-2])
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 40, 32), (33, 1000, 96), (65, 512, 1344), (500, 1536, 512), (1000, 520, 64),
                                    (513, 2304, 768), (2049, 1030, 96), (300, 264, 36), (4000, 2312, 32)])
 def test_fp32(m, n, k):

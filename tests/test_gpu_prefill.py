@@ -39,9 +39,9 @@ def test_gemm_matches_fp32_matmul(m, n, k, dtype):
     torch.testing.assert_close(ob.float().cpu(), ref.to(dtype).float(), atol=1e-2, rtol=1e-2)
 
 
-# Grids of >= 320 tiles of 256 x 384 take the 256 x 384 kernel with its ring
-# of LDS stages: K of 64 (fewer steps than stages), 192 and 2752 (the model's
-# d_ff), ragged M and N. Sampled token rows keep the CPU reference small.
+# Large ragged grids: tiles of 256 x 384 with K of 64 (fewer steps than LDS
+# stages) and 192, and of 128 x 128 at the 324M model's d_ff of 2752. Sampled
+# token rows keep the CPU reference small.
 @pytest.mark.parametrize("m,n,k", [(4100, 8200, 64), (4100, 8200, 192), (2304, 14400, 2752)])
 def test_gemm_large_grid_matches_fp32_matmul(m, n, k):
     g = torch.Generator().manual_seed(m + n + k)
@@ -93,8 +93,8 @@ def _bf16_out(shape, aligned, dtype=torch.bfloat16):
     return out
 
 
-# The bf16 epilogues of the 256 x 384 kernel (q/k/v + RoPE + cache write,
-# SwiGLU, plain bf16 output) with ragged M (token tiles spanning two batch
+# The bf16 epilogues of large grids (q/k/v + RoPE + cache write on 128 x 128
+# tiles, SwiGLU on 256 x 384, plain bf16 output on 256 x 256) with ragged M (token tiles spanning two batch
 # rows), a ragged N, and outputs that are / are not 16-byte aligned.
 @pytest.mark.parametrize("aligned,dtype", [(True, torch.bfloat16), (False, torch.bfloat16), (True, torch.float16)])
 def test_gemm_large_grid_bf16_epilogues(aligned, dtype):
@@ -149,8 +149,8 @@ def test_gemm_large_grid_bf16_epilogues(aligned, dtype):
 
 
 # Head dims that are not multiples of 32: a 32-feature MFMA block then holds
-# two heads (16) or straddles a head boundary (48). The 256 x 384 kernel
-# (large grids), the 128 x 128 one, and for d_model 144 (K % 64 != 0, the
+# two heads (16) or straddles a head boundary (48). Tiles of 256 x 256 (large
+# grids) and 32 x 32 with K split, and for d_model 144 (K % 64 != 0, the
 # q | k | v boundaries inside a 32-feature block) the 16x16 kernel.
 @pytest.mark.parametrize("dk,h,b,t", [(16, 64, 4, 2600), (48, 16, 4, 3500), (16, 8, 2, 100), (48, 3, 3, 70)])
 def test_gemm_qkv_rope_head_dims_across_feature_blocks(dk, h, b, t):
@@ -182,6 +182,13 @@ def test_gemm_qkv_rope_head_dims_across_feature_blocks(dk, h, b, t):
     _ulp_close(f"k cache (RoPE, dk {dk})", kc.cpu()[bi, :, ti], om._round(rot(kr), torch.bfloat16), 2e-3)
     _ulp_close(f"v cache (dk {dk})", vc.cpu()[bi, :, ti], om._round(vr, torch.bfloat16), 2e-3)
     assert not kc[:, :, t:].any() and not vc[:, :, t:].any(), "wrote cache rows past the sequence"
+
+
+@pytest.mark.parametrize("tile,dk,h,b,t", [((128, 128), 16, 64, 4, 2751), ((256, 384), 16, 64, 4, 3451),
+                                           ((128, 128), 48, 16, 4, 2801), ((256, 384), 48, 16, 4, 2501)])
+def test_gemm_qkv_rope_head_dims_on_larger_tiles(tile, dk, h, b, t):
+    assert _lib.gemm_tile(b * t, 3 * dk * h, dk * h, 1)[:2] == tile
+    test_gemm_qkv_rope_head_dims_across_feature_blocks(dk, h, b, t)
 
 
 # d % 4 == 0 and d <= 2048 take the one-wave-per-row kernel (m not a multiple
@@ -223,10 +230,11 @@ def test_rmsnorm_rows_scaled_splits_the_norm(m, d):
 
 
 # The residual GEMM that also prepares the next RMSNorm: x += A W^T, then
-# bf16(x * gain) and per-token sums of x^2 over each 128-feature part, on the
-# 128 x 128 tiles (ragged features, a last part of 64) and the 256 x 384 tiles
-# (ragged tokens and features), with guard rows around every output; N % 8 ==
-# 4 takes the 8-byte stores of the norm input instead of 16-byte ones.
+# bf16(x * gain) and per-token sums of x^2 over each 128-feature part, on
+# 128 x 64 tiles (parts of 128 keep small shapes off the K-split ones; ragged
+# features, a last part of 64) and 256 x 256 tiles (ragged tokens and
+# features), with guard rows around every output; N % 8 == 4 takes the 8-byte
+# stores of the norm input instead of 16-byte ones.
 @pytest.mark.parametrize("m,n,k", [(200, 192, 320), (300, 196, 64), (1000, 1024, 64), (24577, 1088, 128)])
 def test_gemm_residual_norm_and_norm_scale(m, n, k):
     g = torch.Generator().manual_seed(m + n + k + 7)
@@ -595,6 +603,21 @@ def test_prefill_bf16_logits_are_the_rounded_fp32_logits():
     assert torch.equal(model(ids), b16)
     with pytest.raises(TypeError):
         session.prefill(ids, all_logits=True, logits_dtype=torch.float16)
+
+
+def test_a_prompts_logits_in_other_batches_differ_by_less_than_the_format():
+    """A prompt beside others runs on other GEMM tiles, which add its products in another order:
+    its logits move by re-rounded 16-bit values, less than 16-bit storage itself moves them."""
+    cfg = load_model_config("pilot-22m-s256")
+    sd = seeded_state_dict(cfg, 5)
+    model = gpu_model(cfg, sd)
+    ids = seeded_prompt(cfg.vocab_size, 24, 60, 6)
+    alone, beside = model(ids[:1].cuda()).double().cpu()[0], model(ids.cuda()).double().cpu()[0]
+    reference = om.forward(sd, cfg, ids[:1]).double()[0]
+    moved, format_error = (alone - beside).norm().item(), (beside - reference).norm().item()
+    print(f"alone against beside 23 others {moved / reference.norm():.2e}, format {format_error / reference.norm():.2e}")
+    assert _lib.gemm_tile(60, 3 * cfg.d_model, cfg.d_model, 1) != _lib.gemm_tile(24 * 60, 3 * cfg.d_model, cfg.d_model, 1)
+    assert moved <= format_error
 
 
 def test_generate_bf16_uses_prefill_and_matches_step_path():
