@@ -392,7 +392,10 @@ int sfl_rmsnorm_rows_scaled(const float* x, const void* w, void* act_xg, float* 
  * the features f of part p = f / 128 (ceil(n / 128) parts). n % 4 == 0.
  * act_xg must not overlap a (other workgroups may still be reading A while
  * one writes its outputs); each part's sum has a fixed order, so results are
- * the same from call to call. */
+ * the same from call to call. (sfl_prefill_layers takes the form with other
+ * part sizes below, forms the scales in their consumers and gathers the
+ * embedding itself: this entry point, sfl_norm_scale and sfl_embed_rows are for
+ * callers that put a layer together themselves.) */
 int sfl_gemm_residual_norm(const void* a, const void* w, float* x, int m, int n, int k, const void* gain_next,
                            void* act_xg, float* ss_parts, int dtype, void* stream);
 

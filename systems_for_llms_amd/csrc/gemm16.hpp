@@ -209,7 +209,6 @@ __device__ __forceinline__ void store_tile(const GemmArgs& g, const f32x4& v, in
 }
 
 constexpr int K2 = 64;     // K step
-constexpr int TB = 128;    // features and tokens per workgroup
 
 
 template <int TN_, int TM_, int SL_>

@@ -367,8 +367,8 @@ class DecodeSession:
             code, len(w2), b, t, given.shape[1], d, h, f, self.cap, int(fold), float(dk ** -0.5), given.data_ptr(),
             self.tokens.data_ptr(), self.predicted.data_ptr(), self.prompt_len.data_ptr(), self.pos.data_ptr(),
             self.lengths.data_ptr(), self.x.data_ptr(), _weight(model.token_embeddings).data_ptr(),
-            *map(_lib.pointers, weights), self.cos_fm.data_ptr(), self.sin_fm.data_ptr(), x.data_ptr(), act.data_ptr(), q.data_ptr(), attn.data_ptr(), hid.data_ptr(),
-            _lib.ptr(ss), _lib.ptr(scale))
+            *map(_lib.pointers, weights), self.cos_fm.data_ptr(), self.sin_fm.data_ptr(), x.data_ptr(),
+            act.data_ptr(), q.data_ptr(), attn.data_ptr(), hid.data_ptr(), _lib.ptr(ss), _lib.ptr(scale))
         low, high = bounds.tolist()
         if low < 0 or high >= self.vocab:
             raise ValueError("token ids must be in [0, vocab_size)")

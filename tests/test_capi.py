@@ -130,7 +130,8 @@ def test_prefill_layers_refuses_what_its_layers_would_before_any_launch():
                          (dict(fold, attn_norm=odd()), INVALID), (dict(fold, act=20), INVALID),
                          (dict(d_model=96), UNSUPPORTED), (dict(heads=4), UNSUPPORTED), (dict(d_ff=60), UNSUPPORTED),
                          (dict(cos_t=None), INVALID), (dict(sin_t=None), INVALID), (dict(scale=0.0), INVALID),
-                         (dict(scale=float("nan")), INVALID), (dict(f32, act=24), INVALID), (dict(f32, w2=odd()), INVALID),
+                         (dict(scale=float("nan")), INVALID), (dict(f32, act=24), INVALID),
+                         (dict(f32, w2=odd()), INVALID),
                          (dict(f32, batch=1 << 22, seq=2, d_model=48, heads=3), UNSUPPORTED),
                          *((dict({name: second()}), INVALID) for name in ("attn_norm", "w_qkv", "w_out", "ffn_norm",
                                                                          "w13", "w2", "k_cache", "v_cache"))):

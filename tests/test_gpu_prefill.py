@@ -94,8 +94,8 @@ def _bf16_out(shape, aligned, dtype=torch.bfloat16):
 
 
 # The bf16 epilogues of large grids (q/k/v + RoPE + cache write on 128 x 128
-# tiles, SwiGLU on 256 x 384, plain bf16 output on 256 x 256) with ragged M (token tiles spanning two batch
-# rows), a ragged N, and outputs that are / are not 16-byte aligned.
+# tiles, SwiGLU on 256 x 384, plain bf16 output on 256 x 256) with ragged M
+# (token tiles spanning two batch rows), a ragged N, and outputs that are / are not 16-byte aligned.
 @pytest.mark.parametrize("aligned,dtype", [(True, torch.bfloat16), (False, torch.bfloat16), (True, torch.float16)])
 def test_gemm_large_grid_bf16_epilogues(aligned, dtype):
     """The 16-bit epilogues (q/k/v + RoPE + cache, SwiGLU, plain) on the large-grid kernel, in
@@ -615,8 +615,10 @@ def test_a_prompts_logits_in_other_batches_differ_by_less_than_the_format():
     alone, beside = model(ids[:1].cuda()).double().cpu()[0], model(ids.cuda()).double().cpu()[0]
     reference = om.forward(sd, cfg, ids[:1]).double()[0]
     moved, format_error = (alone - beside).norm().item(), (beside - reference).norm().item()
-    print(f"alone against beside 23 others {moved / reference.norm():.2e}, format {format_error / reference.norm():.2e}")
-    assert _lib.gemm_tile(60, 3 * cfg.d_model, cfg.d_model, 1) != _lib.gemm_tile(24 * 60, 3 * cfg.d_model, cfg.d_model, 1)
+    size = reference.norm().item()
+    print(f"alone against beside 23 others {moved / size:.2e}, format {format_error / size:.2e}")
+    tiles = [_lib.gemm_tile(rows, 3 * cfg.d_model, cfg.d_model, 1) for rows in (60, 24 * 60)]
+    assert tiles[0] != tiles[1]
     assert moved <= format_error
 
 
