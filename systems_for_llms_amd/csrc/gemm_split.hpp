@@ -34,9 +34,9 @@ __device__ __forceinline__ f32x16 mma_slot(const u32x4& a, const u32x4& b, f32x1
 // truncation, all of x's sign. Of the nine products of two operands' pieces the
 // eight without p2 p2 are summed in fp32; the one left out is below 2^-30 of
 // the operands' product, under the 2^-24 that an fp32 product rounds by. p0 p0
-// has a sum of its own: the other seven, at most 2^-6 of it, then cost it one
-// rounding in all and not one per product, so a sum of few terms is as exact as
-// one of fp32 products.
+// has a sum of its own: the other seven, about 2^-6 of it at most, then cost it
+// one rounding in all and not one per product, so a sum of few terms is as exact
+// as one of fp32 products.
 // `lost` collects the bits no piece holds in its low half: none for operands
 // of at least 2^-110, some below, where p2 would need values under bf16's
 // smallest subnormal (the MFMAs keep subnormal operands and results); the
